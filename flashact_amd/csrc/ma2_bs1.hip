@@ -11,7 +11,7 @@
 //   SO     all ranks: 24 rows of W_so[:, 96g..96g+96) x attn_g -> partial                      {E}
 //   N_mca  as N_msa with g_msa, b_so                                                            [X]
 //   CQ     ranks 0..5: 16 of the head's 96 q rows x 768, + b_cq                                  [X]
-//   CATT   ranks 0..15: context keys 32r..32r+31 of head g -> normalised partial O + (m, l)    [X]
+//   CATT   rank r: context keys 32r..32r+31 of head g -> normalised partial O + (m, l)          [X]
 //   COMB   token r: combine the key chunks -> attn_g                                            [X]
 //   CO     as SO with W_co                                                                      {E}
 //   N_mlp  as N_msa with g_mca, b_co                                                            [X]
@@ -36,8 +36,10 @@ using namespace fa::ma2att;
 constexpr int D = 768, FF = 3072, AD = 32, QKVN = 3 * D, GUN = 2 * FF;
 constexpr int NX = 8, NR = 32;
 constexpr int TP = 32;   // token slots (Tv <= 32)
-constexpr int KPR = 32;  // context keys per cross-attention rank (Lk <= 512)
-constexpr int MAX_LK = NR / 2 * KPR;
+constexpr int KPR = 32;  // context keys per cross-attention rank
+// Longest context of this kernel: one chunk per rank. (With 16 chunks, Lk = 777 ran on the stage-engine
+// kernel of ma2.hip, whose 12 grid barriers per layer alone cost more than this kernel's layer.)
+constexpr int MAX_LK = NR * KPR;
 
 // ---- workspace (bytes)
 constexpr uint32_t OFF_CTRL = 0;     // u64 seq, u32 err @8, u32 exchange parity bases @12, @16
@@ -53,9 +55,9 @@ constexpr uint32_t X_XN = 0;                          // [32][768] bf16 fragment
 constexpr uint32_t X_QKV = X_XN + TP * D * 2;         // [2][18][64] f32x4 (q | k | v of head g, + bias)
 constexpr uint32_t X_ATT = X_QKV + TP * 288 * 4;      // [32][96] bf16 fragments
 constexpr uint32_t X_QC = X_ATT + TP * HD * 2;        // [2][6][64] f32x4 (+ bias)
-constexpr uint32_t X_CP = X_QC + TP * HD * 4;         // [16 chunks][32][96] bf16 partials
-constexpr uint32_t X_CML = X_CP + 16 * TP * HD * 2;   // [16][32] (m, l) f32
-constexpr uint32_t X_H = X_CML + 16 * TP * 8;         // [32][384] bf16 fragments
+constexpr uint32_t X_CP = X_QC + TP * HD * 4;         // [32 chunks][32][96] bf16 partials
+constexpr uint32_t X_CML = X_CP + NR * TP * HD * 2;   // [32][32] (m, l) f32
+constexpr uint32_t X_H = X_CML + NR * TP * 8;         // [32][384] bf16 fragments
 constexpr uint32_t XB = (X_H + TP * 384 * 2 + 4095) / 4096 * 4096;
 constexpr uint32_t OFF_XCD = OFF_XP + XP_BYTES;
 constexpr uint32_t WS_BYTES = OFF_XCD + NX * XB;
@@ -424,7 +426,7 @@ __device__ __forceinline__ void stage_satt(const Params& p, const Ctx& c) {
   }
 }
 
-// ---- cross attention: context keys 32r..32r+31 of head g (ranks 0..15) --------------------------
+// ---- cross attention: context keys 32r..32r+31 of head g ----------------------------------------
 // kf: K fragments (key tile kt, k-step ks; tile row 4a + i = key 32 r + 8 a + 4 kt + i); vf: V^T
 // fragments (dim tile dt; keys 32 r + 8 lq ..). Both were loaded ahead of the barrier.
 __device__ __forceinline__ void stage_catt(const Params& p, const Ctx& c, const u32x4 (&kf)[2][3], const u32x4 (&vf)[6]) {
@@ -507,28 +509,31 @@ __device__ __forceinline__ void stage_catt(const Params& p, const Ctx& c, const 
 }
 
 // attn_g[token r][d] = sum_c w_c O_c[d], w_c ~ l_c 2^(m_c - M); wave 0, lanes < 48 take dims 2l, 2l+1.
+// NC chunk slots, all their loads in flight together (a loop of 16-chunk trips around the same code
+// slowed the 16-chunk case by 5-11 %, through the waits at the loop's head).
+template <int NC>
 __device__ __forceinline__ void stage_comb(const Params& p, const Ctx& c) {
   const int t = c.r;
   if (t >= p.Tv || c.w != 0) return;
   const int nch = (p.Lk + KPR - 1) / KPR;
   const int d0 = 2 * (c.lane < 48 ? c.lane : 0);
-  u32x2 ml[16];
-  unsigned v[16];
+  u32x2 ml[NC];
+  unsigned v[NC];
 #pragma unroll
-  for (int ch = 0; ch < 16; ch++) {
+  for (int ch = 0; ch < NC; ch++) {
     const int cc = ch < nch ? ch : 0;
     ml[ch] = ldb64<kCpSc1>(c.ws, c.xb + X_CML + (uint32_t)((cc * TP + t) * 8));
     v[ch] = __builtin_amdgcn_raw_buffer_load_b32(c.ws, c.xb + X_CP + (uint32_t)(((cc * TP + t) * HD + d0) * 2), 0, kCpSc1);
   }
   float M = -1e30f;
 #pragma unroll
-  for (int ch = 0; ch < 16; ch++)
+  for (int ch = 0; ch < NC; ch++)
     if (ch < nch) M = fmaxf(M, as_f32(ml[ch][0]));
   float den = 0.f, a0 = 0.f, a1 = 0.f;
 #pragma unroll
-  for (int ch = 0; ch < 16; ch++) {
-    if (ch >= nch) break;
-    const float wc = as_f32(ml[ch][1]) * exp2_w(as_f32(ml[ch][0]) - M);
+  for (int ch = 0; ch < NC; ch++) {
+    if (NC <= 16 && ch >= nch) break;  // (with 32 slots the break kept the loop rolled, its arrays in scratch)
+    const float wc = NC <= 16 || ch < nch ? as_f32(ml[ch][1]) * exp2_w(as_f32(ml[ch][0]) - M) : 0.f;
     den += wc;
     a0 = fmaf(wc, bf_lo(v[ch]), a0);
     a1 = fmaf(wc, bf_hi(v[ch]), a1);
@@ -581,6 +586,9 @@ __device__ __forceinline__ void mark(const Params& p, int idx, uint64_t& t0) {
   }
 }
 
+// NC: context chunk slots of the combine, 16 (Lk <= 512: 10.9 ms per chunk at Lk = 493) or 32 (11.16 ms
+// at Lk = 777, which took 27.6 ms on the stage-engine kernel).
+template <int NC>
 __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
   Ctx c;
   c.g = blockIdx.x & 7;
@@ -722,7 +730,7 @@ __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
       xwait(c);
       mark(p, 15, t0);
       // COMB, with the CO weights in flight
-      stage_comb(p, c);
+      stage_comb<NC>(p, c);
       mark(p, 7, t0);
       xarrive(c);
       u32x4 wco[3];
@@ -802,7 +810,9 @@ int ma2_bs1_launch(const fa_ma2_args* a, fa_stream_t stream) {
   if (a->workspace_bytes < WS_BYTES)
     return host::fail(FA_ERR_INVALID_ARG, "fa_ma2_flow: workspace_bytes=%zu < required %u", a->workspace_bytes,
                       (unsigned)WS_BYTES);
-  int rc = host::check_device((const void*)ma2x_kernel, NTHR, LDS_BYTES, NWG, "fa_ma2_flow");
+  // Up to 512 keys the combine's sixteen chunk slots are enough (half the loads); past that, 32.
+  const void* kern = a->Lk <= NR / 2 * KPR ? (const void*)ma2x_kernel<NR / 2> : (const void*)ma2x_kernel<NR>;
+  int rc = host::check_device(kern, NTHR, LDS_BYTES, NWG, "fa_ma2_flow");
   if (rc != FA_OK) return rc;
   Params p;
   p.w_qkv = static_cast<const bf16*>(a->w_qkv);
@@ -837,7 +847,7 @@ int ma2_bs1_launch(const fa_ma2_args* a, fa_stream_t stream) {
   p.adim = a->adim;
   p.S = a->num_steps;
   void* args[] = {&p};
-  return host::coop_launch((const void*)ma2x_kernel, NWG, NTHR, args, LDS_BYTES, stream, "fa_ma2_flow");
+  return host::coop_launch(kern, NWG, NTHR, args, LDS_BYTES, stream, "fa_ma2_flow");
 }
 
 }  // namespace fa

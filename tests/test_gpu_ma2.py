@@ -38,7 +38,7 @@ def test_ma2_config4_bs1(gpu):
     _check(C.make_case(NL=36, Lk=493, Tv=30, S=10), gpu)
 
 
-# Batch 1 runs the XCD-local kernel up to Tv = 32 and Lk = 512: (1, 512, 32) fills every token lane
+# Batch 1 runs the XCD-local kernel up to Tv = 32 and Lk = 1024: (1, 512, 32) fills every token lane
 # and context rank; (1, 65, 17) leaves one token in the second token tile and a ragged key chunk.
 # (1, 300, 40) runs the generic kernel's small-tile path with four waves per cross-attention item.
 @pytest.mark.parametrize("B,Lk,Tv,S,adim", [(1, 1, 1, 2, 6), (2, 700, 64, 1, 32), (3, 37, 17, 2, 5),
@@ -46,6 +46,15 @@ def test_ma2_config4_bs1(gpu):
                                             (1, 65, 17, 2, 7), (1, 300, 40, 2, 6)])
 def test_ma2_edge_shapes(gpu, B, Lk, Tv, S, adim):
     _check(C.make_case(NL=2, Lk=Lk, Tv=Tv, S=S, adim=adim, batch=B, seed=Lk + Tv), gpu)
+
+
+# Contexts past 512 rows at batch 1: one key in the 17th chunk (513), a ragged chunk (777), every rank
+# attending (1024) and the first context of the stage-engine kernel. Two steps: one Euler step of
+# dt = 1 with unit gates sits at 2e-3 mean-abs from its bf16 operands alone (the stage-engine kernel
+# 2.3e-3 at Lk = 1025, Tv = 5), two at 1.5e-3.
+@pytest.mark.parametrize("Lk,Tv", [(513, 30), (777, 17), (1024, 32), (1025, 5)])
+def test_ma2_long_context(gpu, Lk, Tv):
+    _check(C.make_case(NL=2, Lk=Lk, Tv=Tv, S=2, seed=Lk), gpu)
 
 
 def test_ma2_batch16(gpu):
