@@ -43,8 +43,9 @@ constexpr unsigned kSpinCap = 1u << 20;
 // Workspace rules shared by every kernel of the library, so that one workspace may serve any mix
 // of entry points and shapes:
 //  * Bytes [0, kWsDataBase) hold only control words (u64 launch sequence @0, u32 error bits @8,
-//    u32 exchange parity bases @12 and @16, u32 owner @kWsOwner), u64 epoch flags and the split-K
-//    fixup counters. Every kernel keeps its data at kWsDataBase and above.
+//    u32 exchange parity bases @12 and @16, u32 owner @kWsOwner, u32 finished groups @24, zero at
+//    rest), u64 epoch flags, the split-K fixup counters and the u64 epoch flags that groups of XCDs read
+//    from one another. Every kernel keeps its data at kWsDataBase and above.
 //  * Epoch flags derive from the launch sequence (epoch = seq << 32 + n), so a flag left by any
 //    earlier launch lies below every epoch of the current one.
 //  * Fixup counters are zero at rest (the last arriver resets its counter).
@@ -55,9 +56,10 @@ constexpr unsigned kSpinCap = 1u << 20;
 constexpr uint32_t kWsOwner = 20;
 constexpr uint32_t kWsCounters = 12288;  // [1024] u32
 constexpr uint32_t kWsMaxCounters = 1024;
-constexpr uint32_t kWsDataBase = 16384;
+constexpr uint32_t kWsGroupFlags = 16384;  // [8 XCD][32 rank][4 wave] u64
+constexpr uint32_t kWsDataBase = 24576;
 constexpr unsigned kOwnerPi05Bs1 = 1, kOwnerPi05Batched = 2, kOwnerMa2Bs1 = 3, kOwnerMa2Generic = 4,
-                   kOwnerPrefill = 5;
+                   kOwnerPrefill = 5, kOwnerPi05Group = 6;
 
 __device__ __forceinline__ rsrc_t make_rsrc(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, kRsrcWord3);

@@ -37,6 +37,13 @@ int check_device(const void* kernel, int threads, unsigned lds_bytes, int nwg, c
 // Batched pi0.5 launch (batch >= 2), dispatched from fa_pi05_denoise after the shared checks.
 size_t pi05_batched_workspace_bytes(int batch, int Tv, int Lmax);
 int pi05_denoise_batched(const fa_pi05_args* a, fa_stream_t stream);
+// Refuses what the batched launches refuse (tokens, cache range, traces); both kernels behind it.
+int pi05_check_batched(const fa_pi05_args* a);
+
+// Batches of 2 to 16 samples on groups of XCDs (pi05_group.hip).
+bool pi05_group_eligible(int batch, int Tv);
+size_t pi05_group_workspace_bytes(int batch);
+int pi05_denoise_group(const fa_pi05_args* a, fa_stream_t stream);
 
 // K/V hand-off (srows > 0): enqueues the de-interleave / transpose of kvsrc_k / kvsrc_v into the
 // caches ahead of the denoise launch. Arguments are checked by fa_pi05_denoise.

@@ -355,7 +355,7 @@ size_t pi05_batched_workspace_bytes(int batch, int Tv, int Lmax) {
   return n < 0xffffffffull ? n : 0;
 }
 
-int pi05_denoise_batched(const fa_pi05_args* a, fa_stream_t stream) {
+int pi05_check_batched(const fa_pi05_args* a) {
   using namespace fa::pb;
   if ((size_t)a->batch * a->Tv > (size_t)MAX_TOKENS)
     return host::fail(FA_ERR_INVALID_ARG, "fa_pi05_denoise: batch x Tv = %d exceeds %d tokens", a->batch * a->Tv,
@@ -370,6 +370,11 @@ int pi05_denoise_batched(const fa_pi05_args* a, fa_stream_t stream) {
                       cache_bytes);
   if (a->trace)
     return host::fail(FA_ERR_UNSUPPORTED, "fa_pi05_denoise: per-wave traces exist for batch 1 only");
+  return FA_OK;
+}
+
+int pi05_denoise_batched(const fa_pi05_args* a, fa_stream_t stream) {
+  using namespace fa::pb;
   Params p;
   p.w1 = static_cast<const bf16*>(a->w1);
   p.wo = static_cast<const bf16*>(a->wo);

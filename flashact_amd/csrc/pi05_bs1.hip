@@ -47,6 +47,7 @@
 #include "../../include/flashact_mi355x.h"
 #include "fa_host.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace fa {
@@ -1335,7 +1336,8 @@ using namespace fa;
 extern "C" size_t fa_pi05_workspace_bytes(int batch, int Tv, int Lmax) {
   if (batch == 1) return pi05::WS_BYTES;
   if (batch < 1 || batch > fa_pi05_max_batch()) return 0;
-  return pi05_batched_workspace_bytes(batch, Tv, Lmax);
+  const size_t n = pi05_batched_workspace_bytes(batch, Tv, Lmax);
+  return n && pi05_group_eligible(batch, Tv) ? std::max(n, pi05_group_workspace_bytes(batch)) : n;
 }
 
 extern "C" int fa_pi05_max_batch(void) { return 64; }
@@ -1453,7 +1455,15 @@ extern "C" int fa_pi05_denoise(const fa_pi05_args* a, fa_stream_t stream) {
   if (a->cache_dtype != FA_DTYPE_BF16 && !kv16)
     return host::fail(FA_ERR_INVALID_ARG, "fa_pi05_denoise: cache_dtype=%d is neither FA_DTYPE_BF16 nor FA_DTYPE_F16",
                       a->cache_dtype);
-  if (a->batch > 1) return pi05_denoise_batched(a, stream);
+  if (a->batch > 1) {
+    const int rc = pi05_check_batched(a);
+    if (rc != FA_OK) return rc;
+    // Up to 16 samples, groups of XCDs; past that (or in a workspace too small for the groups) the
+    // stage engine, whose GEMM tiles are then full.
+    if (pi05_group_eligible(a->batch, a->Tv) && a->workspace_bytes >= pi05_group_workspace_bytes(a->batch))
+      return pi05_denoise_group(a, stream);
+    return pi05_denoise_batched(a, stream);
+  }
   if (a->workspace_bytes < WS_BYTES)
     return host::fail(FA_ERR_INVALID_ARG, "fa_pi05_denoise: workspace_bytes=%zu < required %u", a->workspace_bytes,
                       (unsigned)WS_BYTES);
@@ -1509,7 +1519,9 @@ extern "C" int fa_pi05_denoise_noalloc(const fa_pi05_args* a, fa_stream_t stream
   if (a->workspace || a->workspace_bytes)
     return host::fail(FA_ERR_INVALID_ARG, "fa_pi05_denoise_noalloc: workspace must be NULL / 0 (this entry point "
                                           "uses the library's static scratch)");
-  const size_t need = fa_pi05_workspace_bytes(a->batch, a->Tv, a->Lmax);
+  // (a batched request that fits runs on the stage engine where the group kernel's workspace does not)
+  const size_t need = a->batch > 1 && a->batch <= fa_pi05_max_batch() ? pi05_batched_workspace_bytes(a->batch, a->Tv, a->Lmax)
+                                                                   : fa_pi05_workspace_bytes(a->batch, a->Tv, a->Lmax);
   if (need == 0 || need > kNoAllocScratchBytes)
     return host::fail(FA_ERR_INVALID_ARG, "fa_pi05_denoise_noalloc: batch=%d Tv=%d Lmax=%d needs a %zu-byte workspace; "
                       "the static scratch holds %zu bytes (use fa_pi05_denoise with a caller workspace)",

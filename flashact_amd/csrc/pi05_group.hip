@@ -1,0 +1,1179 @@
+// pi0.5 action-expert denoise loop for 2 to 16 samples: groups of XCDs, each group running its own
+// samples through the whole S-step Euler loop with no grid-wide barrier. ONE cooperative launch of 256
+// workgroups (one per CU) of 6 waves.
+//
+// G XCDs form a group (G = 4: 2 groups, G = 2: 4, G = 1: 8) of up to NB samples (NB = 1 or 2).
+// XCD j of a group owns query heads [8/G j, 8/G (j + 1)), MLP columns [4096/G j, ..) and those K windows
+// of the O and down projections, so everything but the projections' partial sums stays in its L2.
+// Within the XCD, rank r = blockIdx / 8 owns output rows of every GEMM; the O and down projections are
+// also split over C = 4/G K windows of 512 / 1024, so a rank reads a quarter of the token operand instead
+// of all of it, and every group ends with 4 partial sums per residual update (the K split of the
+// stage-engine kernel, pi05_batched.hip).
+// Waves 0-3 compute: wave w owns tokens 16w..16w+15 of each of the group's samples in every stage (NB
+// token tiles) and signals its own flags, so no workgroup barrier runs after the prologue. Waves 4-5
+// load: they stream the CU's weight rows and its chunk's prefix K/V from HBM into an 8-page LDS ring
+// (16 KB pages), free-running ahead of the compute waves.
+//
+// Per layer ([W] = waits for the waves that wrote the operand, [X] = XCD barrier, {E} = waits for the
+// group's partial sums):
+//   N1   x += gate * sum of the 4 down partials (layer 0: x = embed(x_t)); xn = adaRMS(x)   (x in LDS)
+//   [W] QKV   2048/G + 512 rows (heads of the XCD, all k and v), RoPE
+//   [X] ATT   item = (sample, head, key chunk), 32 items: prefix keys from the ring, this step's keys
+//             spread over the chunks
+//   [W] COMB  key chunks combined, one operand fragment at a time
+//   [W] O     partial sums {E} N2 [W] GU [W] DN partial sums {E}
+//
+// What bounds it: each group streams all 34.6 MB of a layer's weights, 34.6/G MB per XCD. The fabric
+// feeds one XCD at 0.85-0.95 TB/s while all eight read (1.0 with four, 1.34 alone): 37 us per layer with
+// G = 1, 19 with G = 2, 10 with G = 4. The stage engine at these batches had 40 to 180 GEMM items for the 256
+// CUs in every stage but gate/up, and eight grid barriers of about 2 us per layer.
+#include "fa_device.h"
+#include "../../include/flashact_mi355x.h"
+#include "fa_host.h"
+
+namespace fa {
+namespace pg {
+
+constexpr int D = 1024, HD = 256, AD = 32, FF = 4096, QD = 2048;
+constexpr int NX = 8, NR = 32, NWG = 256, TP = 64;
+constexpr int NCW = 4, NLW = 2, NTH = 64 * (NCW + NLW);  // compute waves, loader waves
+constexpr int RING = 8, PAGE = 16384;                   // ring pages, page bytes
+constexpr int MAXF = 2;                                 // pages in flight per loader wave (1: 3-9 % slower)
+constexpr uint32_t OOB = 0x80000000u;                   // buffer offset past every resource
+
+// Shape of one configuration: G XCDs per group, NB samples per group.
+template <int G_, int NB_>
+struct Cfg {
+  static constexpr int G = G_, NB = NB_;
+  static constexpr int NGRP = NX / G;
+  static constexpr int HX = 8 / G;             // heads per XCD
+  static constexpr int C = 4 / G;              // K windows of the O and down projections per XCD
+  static constexpr int NKC = NR / (NB * HX);   // key chunks per (sample, head)
+  static constexpr int SK = TP / NKC;          // this step's keys per chunk
+  static constexpr int SKT = SK > 16 ? 2 : 1;  // their key tiles (tile kt holds keys 8 a + 4 kt + i, see below)
+  static constexpr int SEGU = NKC >= 16 ? 1 : 2;  // 64-key units per attention segment
+  static constexpr int RQ = (QD / G + 512) / (16 * NR);  // row tiles per rank: QKV
+  static constexpr int RP = D * C / (16 * NR);           // O and down
+  static constexpr int RG = 2 * FF / G / (16 * NR);      // gate/up, in PG passes of RGP
+  static constexpr int PG = RG > 8 ? 2 : 1, RGP = RG / PG;
+  static constexpr int KO = 16, KD = 32, KX = 32;  // k-steps: O window, down window, QKV and gate/up
+  static constexpr int PQ = RQ * KX / 16, PO = RP * KO / 16, PGU = RG * KX / 16, PD = RP * KD / 16;  // pages
+  static constexpr int FPR = NB * HX / 4;      // combine fragments per wave (0: ranks < 16 take one)
+  // workspace of one XCD (bytes), operands in MFMA fragment order [tile (n, w)][k-step][1 KB]
+  static constexpr uint32_t X_XN = 0;
+  static constexpr uint32_t X_Q = X_XN + NB * TP * D * 2;             // [n][head][w][8 k-steps]
+  static constexpr uint32_t X_ATTP = X_Q + NB * HX * TP * HD * 2;     // [rank][w][8 k-steps]
+  static constexpr uint32_t X_ML = X_ATTP + NR * TP * HD * 2;         // [rank][64] (m, l)
+  static constexpr uint32_t X_ATTN = X_ML + NR * TP * 8;              // [n, w][8 HX k-steps]
+  static constexpr uint32_t X_H = X_ATTN + NB * TP * HX * HD * 2;     // [n, w][128 / G k-steps]
+  static constexpr uint32_t X_KS = X_H + NB * TP * (FF / G) * 2;      // [layer parity][n][64][256]
+  static constexpr uint32_t X_VS = X_KS + 2 * NB * TP * HD * 2;       // [layer parity][n][256][64]
+  static constexpr uint32_t XB = X_VS + 2 * NB * TP * HD * 2;
+  static constexpr uint32_t OFF_XCD = kWsDataBase;
+  // fp32 partial sums [O | down][4 windows][NB 64 tokens][1024] of one group; one buffer serves both with
+  // G = 1, where the down projection starts only after every reader of the O partials is done
+  static constexpr uint32_t PB1 = 4u * NB * TP * D * 4, PB = (G == 1 ? 1 : 2) * PB1;
+  static constexpr uint32_t OFF_PART = OFF_XCD + NX * XB;
+  static constexpr uint32_t WS = OFF_PART + NGRP * PB;
+  // LDS (bytes)
+  static constexpr uint32_t L_CTL = RING * PAGE;           // u32 ready[2], consumed[4], abort
+  static constexpr uint32_t L_XRES = L_CTL + 64;           // f32 [2 NB][1024] residual rows
+  static constexpr uint32_t L_XT = L_XRES + 2 * NB * D * 4;  // f32 [2 NB][32] x_t rows
+  static constexpr uint32_t LDS = L_XT + 2 * NB * AD * 4;
+  static_assert(LDS <= 160 * 1024, "LDS of one CU");
+  static_assert(NB * HX * NKC == NR && NKC >= 2 && NB <= 2, "one attention item per rank");
+};
+constexpr uint32_t OFF_CTRL = 0, OFF_XFLAG = 1024;
+constexpr uint32_t OFF_DONE = 24;  // u32: groups of this launch that have finished
+static_assert(OFF_XFLAG + NX * NR * NCW * 8 <= kWsCounters, "flags stay below the fixup counters");
+static_assert(kWsGroupFlags + NX * NR * NCW * 8 <= kWsDataBase, "group flags stay below the data");
+
+__host__ __device__ constexpr uint32_t frag_off(int KS, int t, int k) {  // as in pi05_bs1.hip
+  return (uint32_t)(((((t >> 4) * KS + (k >> 5)) * 16 + (t & 15)) * 4 + ((k >> 3) & 3)) * 16 + (k & 7) * 2);
+}
+
+struct Params {
+  const bf16* w1;
+  const bf16* wo;
+  const bf16* w2;
+  const bf16* w3;
+  const float* mods;
+  const float* mod_final;
+  const float* rope_cos;
+  const float* rope_sin;
+  const float* w_ain;
+  const float* b_ain;
+  const float* w_aout;
+  const float* b_aout;
+  bf16* kcache;
+  bf16* vtcache;
+  float* x_t;
+  unsigned long long* stage_cycles;
+  unsigned char* ws;
+  int NL, Lp, Lmax, S, Tv, B, xt_rows;
+};
+
+extern __shared__ __attribute__((aligned(16))) unsigned char fg_lds[];
+
+struct Ctx {
+  int x, j, grp, r, wave, lane, lr, lq;
+  int ns;                 // samples of this group
+  int an, ah, kbeg, kend, sbeg, nsfx, nun;  // attention item: slot, head, prefix keys, this step's keys, 64-key units
+  rsrc_t ws, rc, rs;
+  uint32_t xb, part;      // byte offsets of this XCD's block and this group's partial sums
+  uint32_t lds_addr;
+  unsigned* err;
+  uint64_t e, eg;         // epochs of this wave's latest XCD / group signal
+};
+
+// Recompute lane-derived addresses per stage instead of keeping them live across the layer.
+__device__ __forceinline__ void launder(Ctx& c) { asm volatile("" : "+v"(c.lane), "+v"(c.lr), "+v"(c.lq)); }
+
+template <class K>
+__device__ __forceinline__ unsigned ctl_ld(int i) {
+  return __hip_atomic_load(reinterpret_cast<unsigned*>(fg_lds + K::L_CTL) + i, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+template <class K>
+__device__ __forceinline__ void ctl_st(int i, unsigned v) {
+  __hip_atomic_store(reinterpret_cast<unsigned*>(fg_lds + K::L_CTL) + i, v, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ bool aborted(const Ctx& c) {
+  return __hip_atomic_load(c.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kErrSpin;
+}
+
+// ---------------------------------------------------------------- synchronisation
+// Signal: the wave drains its stores and publishes its epoch to its own flag (plain store, read by its
+// XCD). Waits are capped and set the sticky error bit, which makes every later wait return at once.
+__device__ __forceinline__ void xcd_signal(const Params& p, Ctx& c) {
+  __builtin_amdgcn_s_waitcnt(0);
+  c.e += 1;
+  if (c.lane == 0)
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(p.ws + OFF_XFLAG) + (c.x * NR + c.r) * NCW + c.wave, c.e,
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// Waits until ready(lane) holds in every lane of the wave; `load` returns whether the lane's flags are.
+template <class F>
+__device__ __forceinline__ void poll(const Ctx& c, const F& ok) {
+  if (aborted(c)) return;
+  for (unsigned it = 0;; ++it) {
+    if (__builtin_amdgcn_ballot_w64(!ok()) == 0) break;
+    if (it > kSpinCap) {
+      if (c.lane == 0) atomicOr(c.err, kErrSpin);
+      break;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+  asm volatile("" ::: "memory");  // loads after the wait stay after it
+}
+__device__ __forceinline__ bool flag_ge(u32x2 v, uint64_t e) { return (((uint64_t)v[1] << 32) | v[0]) >= e; }
+
+__device__ __forceinline__ void xcd_sync(const Params& p, Ctx& c) {
+  xcd_signal(p, c);
+  const uint32_t off = OFF_XFLAG + c.x * (NR * NCW * 8) + c.lane * 16;
+  poll(c, [&] {
+    const u32x4 v = ldb128<kCpSc1>(c.ws, off);
+    return flag_ge(u32x2{v[0], v[1]}, c.e) && flag_ge(u32x2{v[2], v[3]}, c.e);
+  });
+}
+// Waits until this wave index of the ranks in `mask` has passed the sync point this wave passed last.
+__device__ __forceinline__ void xcd_wait(const Ctx& c, uint32_t mask) {
+  const bool mine = c.lane < NR && ((mask >> (c.lane & 31)) & 1u);
+  const uint32_t off = mine ? OFF_XFLAG + ((c.x * NR + c.lane) * NCW + c.wave) * 8 : OOB;
+  poll(c, [&] { return !mine || flag_ge(ldb64<kCpSc1>(c.ws, off), c.e); });
+}
+// Token t of a sample is normed by rank t % 32, wave t / 16: the norm waves of this wave's tile.
+__device__ __forceinline__ void wait_norm_rows(const Ctx& c) { xcd_wait(c, c.wave & 1 ? 0xffff0000u : 0xffffu); }
+
+// Partial sums: published to the whole group. With G = 1 that is the XCD; otherwise the stores went out
+// with sc1 and so does the flag (its own array, read across XCDs).
+template <class K>
+__device__ __forceinline__ void part_signal(const Params& p, Ctx& c) {
+  if constexpr (K::G == 1) {
+    xcd_signal(p, c);
+  } else {
+    __builtin_amdgcn_s_waitcnt(0);
+    c.eg += 1;
+    if (c.lane == 0)
+      __hip_atomic_store(reinterpret_cast<uint64_t*>(p.ws + kWsGroupFlags) + (c.x * NR + c.r) * NCW + c.wave, c.eg,
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+template <class K>
+__device__ __forceinline__ void part_wait(const Ctx& c) {
+  if constexpr (K::G == 1) {
+    xcd_wait(c, 0xffffffffu);
+  } else {
+    const uint32_t off = kWsGroupFlags + ((c.grp * K::G * NR + c.lane) * NCW + c.wave) * 8;
+    poll(c, [&] {
+      u32x2 v[K::G / 2];
+#pragma unroll
+      for (int i = 0; i < K::G / 2; i++) v[i] = ldb64<kCpSc1>(c.ws, off + i * 64 * NCW * 8);
+      bool ok = true;
+#pragma unroll
+      for (int i = 0; i < K::G / 2; i++) ok = ok && flag_ge(v[i], c.eg);
+      return ok;
+    });
+  }
+}
+// cache policy of partial-sum stores: they leave the XCD only with G > 1
+template <class K>
+constexpr int kCpPart = K::G == 1 ? kCpPlain : kCpSc1;
+
+// ---------------------------------------------------------------- weight ring
+template <class K>
+__device__ __forceinline__ void page_wait(const Ctx& c, int pg) {
+  for (unsigned it = 0;; ++it) {
+    const unsigned r0 = ctl_ld<K>(0), r1 = ctl_ld<K>(1);
+    if ((int)min(r0, r1) > pg || ctl_ld<K>(6)) break;
+    if (it > kSpinCap) {
+      ctl_st<K>(6, 1u);
+      if (c.lane == 0) atomicOr(c.err, kErrSpin);
+      break;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+  asm volatile("" ::: "memory");
+}
+template <class K>
+__device__ __forceinline__ void page_release(const Ctx& c, int upto) {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's LDS reads have returned
+  if (c.lane == 0) ctl_st<K>(2 + c.wave, (unsigned)upto);
+}
+
+// global_load_lds_dwordx4 with a wave-uniform base and a 32-bit lane offset: lane i copies 16 bytes to
+// LDS m0 + 16 i, so a fragment lands in MFMA lane order.
+__device__ __forceinline__ void dma16(const unsigned char* base, uint32_t voff, uint32_t lds) {
+  unsigned saved;
+  // (each half is cast to uint32_t before widening: readfirstlane returns int)
+  const uint64_t a = reinterpret_cast<uint64_t>(base);
+  const uint64_t u = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32)) << 32 |
+                     (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a);
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+               : "=&s"(saved)
+               : "v"(voff), "s"(u), "s"(__builtin_amdgcn_readfirstlane(lds))
+               : "memory");
+}
+
+// First row of QKV row tile rt of rank r (virtual rows: this XCD's heads, then k, then v).
+template <class K>
+__device__ __forceinline__ int qkv_row(int j, int vr) {
+  return vr < 256 * K::HX ? 256 * K::HX * j + vr : QD + (vr - 256 * K::HX);
+}
+
+#define FA_PG_VMCNT(n) (((n) & 15) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
+
+// Loader wave lw copies fragments 8 lw .. 8 lw + 7 of every page. Pages go out in the order the compute
+// waves read them: QKV, the chunk's K and V^T blocks, O, gate/up (PG passes), down; fragment F of a GEMM
+// stage with R row tiles is (k-step F / R, row tile F % R). A page needs its ring slot released by the
+// four compute waves and at most MAXF of this wave's pages in flight.
+template <class K>
+struct Loader {
+  const Params& p;
+  const Ctx& c;
+  int lw, pg = 0, done = 0;
+  bool ok = true;
+
+  __device__ __forceinline__ void complete_oldest() {
+    if (pg - done > 1)  // another page is in flight behind the oldest
+      __builtin_amdgcn_s_waitcnt(FA_PG_VMCNT(8));
+    else
+      __builtin_amdgcn_s_waitcnt(FA_PG_VMCNT(0));
+    static_assert(MAXF <= 2, "waits cover two pages in flight");
+    asm volatile("" ::: "memory");
+    ++done;
+    if (c.lane == 0) ctl_st<K>(lw, (unsigned)done);
+  }
+  __device__ __forceinline__ bool room() {
+    for (unsigned idle = 0;;) {
+      if (pg - done < MAXF) {
+        if (pg < RING) return true;
+        const unsigned m = min(min(ctl_ld<K>(2), ctl_ld<K>(3)), min(ctl_ld<K>(4), ctl_ld<K>(5)));
+        if ((int)m >= pg - RING + 1) return true;
+      }
+      if (done < pg) {
+        complete_oldest();
+        idle = 0;
+        continue;
+      }
+      if (ctl_ld<K>(6) || ++idle > kSpinCap) {
+        if (!ctl_ld<K>(6)) {
+          ctl_st<K>(6, 1u);
+          if (c.lane == 0) atomicOr(c.err, kErrSpin);
+        }
+        ok = false;
+        return false;
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
+  }
+  __device__ __forceinline__ uint32_t dst() const { return c.lds_addr + (uint32_t)(pg % RING) * PAGE + lw * 8192; }
+
+  // R row tiles of one GEMM stage: base(rt) = the tile's first row at the stage's first k
+  template <int R, int NP, class Base>
+  __device__ __forceinline__ void stage(uint32_t voff, const Base& base) {
+#pragma unroll 1
+    for (int i = 0; i < NP && ok; i++) {
+      if (!room()) return;
+      const uint32_t d = dst();
+#pragma unroll
+      for (int f = 0; f < 8; f++) {
+        const int F = 16 * i + 8 * lw + f, ks = F / R, rt = F - ks * R;
+        dma16(base(rt) + ks * 64, voff, d + f * 1024);
+      }
+      pg++;
+    }
+  }
+
+  __device__ void run() {
+    const int NL = p.NL;
+    const uint32_t vq = c.lr * (D * 2) + c.lq * 16, vo = c.lr * (QD * 2) + c.lq * 16, vd = c.lr * (FF * 2) + c.lq * 16;
+    const int win = c.r / (NR / K::C), rg = c.r % (NR / K::C);  // K window and row group of O and down
+    const int b = c.grp + c.an * K::NGRP;
+    const uint32_t vstep = 16u * p.Lmax * 2;
+    auto u8 = [](const bf16* q) { return reinterpret_cast<const unsigned char*>(q); };
+#pragma unroll 1
+    for (int li = 0; li < p.S * NL && ok; li++) {
+      const int l = li % NL;
+      const unsigned char* w1 = u8(p.w1) + (size_t)l * 2560 * D * 2;
+      stage<K::RQ, K::PQ>(vq, [&](int rt) { return w1 + (size_t)qkv_row<K>(c.j, 16 * (K::RQ * c.r + rt)) * D * 2; });
+      const unsigned char* kb = u8(p.kcache) + ((size_t)b * NL + l) * p.Lmax * HD * 2;
+      const unsigned char* vb = u8(p.vtcache) + ((size_t)b * NL + l) * HD * p.Lmax * 2;
+#pragma unroll 1
+      for (int u0 = 0; u0 < c.nun && ok; u0 += K::SEGU) {  // a segment: its K pages, then its V^T pages
+        const int np = 2 * min(K::SEGU, c.nun - u0);
+#pragma unroll 1
+        for (int i = 0; i < np; i++) {  // K: key tile lw, k-step f; keys past the chunk copy key 0 (masked later)
+          if (!room()) break;
+          int key = c.kbeg + 64 * u0 + 32 * i + 8 * (c.lr >> 2) + 4 * lw + (c.lr & 3);
+          if (key >= c.kend) key = 0;
+          const uint32_t d = dst();
+#pragma unroll
+          for (int f = 0; f < 8; f++) dma16(kb + f * 64, (uint32_t)key * (HD * 2) + c.lq * 16, d + f * 1024);
+          pg++;
+        }
+#pragma unroll 1
+        for (int i = 0; i < np; i++) {  // V^T: dim tile 8 lw + f; an 8-key group that starts in the chunk
+          if (!room()) break;         // stays within the row (Lmax)
+          int kv = c.kbeg + 64 * u0 + 32 * i + 8 * c.lq;
+          if (kv >= c.kend) kv = 0;
+          const uint32_t vv = (uint32_t)c.lr * p.Lmax * 2 + kv * 2;
+          const uint32_t d = dst();
+#pragma unroll
+          for (int f = 0; f < 8; f++) dma16(vb + (size_t)(8 * lw + f) * vstep, vv, d + f * 1024);
+          pg++;
+        }
+      }
+      const unsigned char* wo = u8(p.wo) + ((size_t)l * D * QD + (size_t)16 * K::RP * rg * QD + 512 * (K::C * c.j + win)) * 2;
+      stage<K::RP, K::PO>(vo, [&](int rt) { return wo + (size_t)rt * 16 * QD * 2; });
+#pragma unroll 1
+      for (int q = 0; q < K::PG; q++) {
+        const unsigned char* w2 =
+            u8(p.w2) + ((size_t)l * 2 * FF + (size_t)c.j * (2 * FF / K::G) + 16 * (K::RG * c.r + K::RGP * q)) * D * 2;
+        stage<K::RGP, K::PGU / K::PG>(vq, [&](int rt) { return w2 + (size_t)rt * 16 * D * 2; });
+      }
+      const unsigned char* w3 = u8(p.w3) + ((size_t)l * D * FF + (size_t)16 * K::RP * rg * FF + 1024 * (K::C * c.j + win)) * 2;
+      stage<K::RP, K::PD>(vd, [&](int rt) { return w3 + (size_t)rt * 16 * FF * 2; });
+    }
+    if (ok)
+      while (done < pg) complete_oldest();
+    __builtin_amdgcn_s_waitcnt(0);
+  }
+};
+
+// ---------------------------------------------------------------- GEMM (NB token tiles per wave)
+// acc[n][rt] = W[row tile rt][k] X[token][k] over KS k-steps, weights from ring pages pg0.. (fragment
+// F = ks R + rt), tokens from the workspace at xoff[n] + 1 KB per k-step (OOB: zeros). The operand
+// loads run two chunks of KC k-steps ahead (one chunk's MFMAs take 0.3-0.4 us, less than a loaded L2
+// round trip); A fragments are read from LDS in batches ahead of their MFMAs, each feeding NB of them;
+// pages are released as their last fragment is read.
+template <class K, int R, int KS>
+__device__ __forceinline__ void gemm(f32x4 (&acc)[K::NB][R], const Ctx& c, int pg0, const uint32_t (&xoff)[K::NB]) {
+  constexpr int NB = K::NB, KC = 8 / NB, NCK = KS / KC, NA = KC * R;
+  constexpr int AB = NA % 8 == 0 ? 8 : (NA % 5 == 0 ? 5 : 6);
+  static_assert(NA % AB == 0, "whole batches");
+  constexpr int CH = R * NB >= 4 ? 1 : 2;  // accumulator chains per row tile
+  f32x4 ac[CH][NB][R];
+#pragma unroll
+  for (int h = 0; h < CH; h++)
+#pragma unroll
+    for (int n = 0; n < NB; n++)
+#pragma unroll
+      for (int rt = 0; rt < R; rt++) ac[h][n][rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  u32x4 xf[3][NB][KC];
+  auto load = [&](int ck) __attribute__((always_inline)) {
+#pragma unroll
+    for (int n = 0; n < NB; n++)
+#pragma unroll
+      for (int k = 0; k < KC; k++) xf[ck % 3][n][k] = ldb128<kCpSc1>(c.ws, xoff[n] + (ck * KC + k) * 1024);
+  };
+  load(0);
+  if (NCK > 1) load(1);
+#pragma unroll
+  for (int ck = 0; ck < NCK; ck++) {
+    if (ck + 2 < NCK) load(ck + 2);
+    page_wait<K>(c, pg0 + ((ck + 1) * NA - 1) / 16);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int h = 0; h < NA; h += AB) {
+      u32x4 af[AB];
+#pragma unroll
+      for (int q = 0; q < AB; q++) {
+        const int F = ck * NA + h + q;
+        af[q] = *reinterpret_cast<const u32x4*>(fg_lds + ((pg0 + F / 16) % RING) * PAGE + c.lane * 16 + (F % 16) * 1024);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < AB; q++) {
+        const int k = (h + q) / R, rt = (h + q) % R;
+#pragma unroll
+        for (int n = 0; n < NB; n++) ac[k % CH][n][rt] = mfma16(af[q], xf[ck % 3][n][k], ac[k % CH][n][rt]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if ((ck + 1) * NA / 16 > ck * NA / 16) page_release<K>(c, pg0 + (ck + 1) * NA / 16);
+  }
+#pragma unroll
+  for (int n = 0; n < NB; n++)
+#pragma unroll
+    for (int rt = 0; rt < R; rt++) acc[n][rt] = CH == 2 ? ac[0][n][rt] + ac[CH - 1][n][rt] : ac[0][n][rt];
+}
+
+// Workspace offsets of the wave's token rows (tile (n, w)) of a fragment-ordered operand with KT k-steps,
+// from k-step ks0; rows past Tv or of an absent sample read zeros.
+template <class K>
+__device__ __forceinline__ void tok_off(const Params& p, const Ctx& c, uint32_t base, int KT, int ks0, uint32_t (&o)[K::NB]) {
+  const int t = 16 * c.wave + c.lr;
+#pragma unroll
+  for (int n = 0; n < K::NB; n++)
+    o[n] = t < p.Tv && n < c.ns ? c.xb + base + (uint32_t)(((n * 4 + c.wave) * KT + ks0) * 1024 + (c.lr * 4 + c.lq) * 16) : OOB;
+}
+
+// ---------------------------------------------------------------- norm stages
+// MODE 0: x = embed(x_t). MODE 1: x += gate * sum of the 4 partials. MODE 2: as 1, then the final norm, the
+// action projection and the Euler update. The wave norms token t = r + 32 (wave / 2) of every sample
+// (LDS slot 2 n + wave / 2); lane holds columns 4 lane + 256 k + i.
+template <class K, int MODE>
+__device__ __forceinline__ void stage_norm(const Params& p, const Ctx& c, uint32_t part, const float* gate,
+                                           const float* scale, const float* shift, float dt) {
+  const int t = c.r + 32 * (c.wave >> 1);
+  // the modulations do not depend on the wait; the partials of every sample are requested together
+  f32x4 sc[4], sh[4], gt[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const int d = 4 * c.lane + 256 * k;
+    sc[k] = *reinterpret_cast<const f32x4*>(scale + d);
+    sh[k] = *reinterpret_cast<const f32x4*>(shift + d);
+    if (MODE != 0) gt[k] = *reinterpret_cast<const f32x4*>(gate + d);
+  }
+  u32x4 v[K::NB][4][4];
+  if (MODE != 0) {
+    part_wait<K>(c);
+#pragma unroll
+    for (int n = 0; n < K::NB; n++)
+#pragma unroll
+      for (int s = 0; s < 4; s++)
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+          v[n][s][k] = ldb128<kCpSc1>(c.ws, c.part + part + (uint32_t)(((n * TP + t) * D + 4 * c.lane) * 4) + s * (K::PB1 / 4) + k * 1024);
+  }
+#pragma unroll
+  for (int n = 0; n < K::NB; n++) {
+    if (n >= c.ns) continue;
+    float* xres = reinterpret_cast<float*>(fg_lds + K::L_XRES) + (2 * n + (c.wave >> 1)) * D;
+    float* xt = reinterpret_cast<float*>(fg_lds + K::L_XT) + (2 * n + (c.wave >> 1)) * AD;
+    f32x4 x[4];
+    if (MODE == 0) {
+      // coalesced 1 KB reads of W_ain [1024][32]: read j covers rows 8j..8j+7 (lane L: row 8j + L/8,
+      // inputs 4 (L%8)..+3), an 8-lane DPP sum finishes each row
+      const f32x4 xa = *reinterpret_cast<const f32x4*>(xt + 4 * (c.lane & 7));
+      const float* W = p.w_ain + 4 * c.lane;
+#pragma unroll 1
+      for (int j0 = 0; j0 < D / 8; j0 += 8) {
+        f32x4 w[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) w[q] = *reinterpret_cast<const f32x4*>(W + (size_t)(j0 + q) * 8 * AD);
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+          float s = w[q][0] * xa[0] + w[q][1] * xa[1] + w[q][2] * xa[2] + w[q][3] * xa[3];
+          s = dpp_f32<0xB1>(s) + s;
+          s = dpp_f32<0x4E>(s) + s;
+          s = dpp_f32<0x141>(s) + s;
+          if ((c.lane & 7) == 0) xres[8 * (j0 + q) + (c.lane >> 3)] = s;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const int d = 4 * c.lane + 256 * k;
+        x[k] = *reinterpret_cast<const f32x4*>(xres + d) + *reinterpret_cast<const f32x4*>(p.b_ain + d);
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const f32x4 s = as_f32x4(v[n][0][k]) + as_f32x4(v[n][1][k]) + as_f32x4(v[n][2][k]) + as_f32x4(v[n][3][k]);
+        x[k] = *reinterpret_cast<const f32x4*>(xres + 4 * c.lane + 256 * k) + gt[k] * s;
+      }
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; k++) ss += x[k][0] * x[k][0] + x[k][1] * x[k][1] + x[k][2] * x[k][2] + x[k][3] * x[k][3];
+    const float rr = rsqrtf(wave_sum(ss) / (float)D + 1e-6f);
+    f32x4 h[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) h[k][i] = x[k][i] * rr * (1.0f + sc[k][i]) + sh[k][i];
+    if (MODE != 2) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const int d = 4 * c.lane + 256 * k;
+        *reinterpret_cast<f32x4*>(xres + d) = x[k];
+        // whole 16-byte slots: lanes (2i, 2i + 1) hold columns 8i .. 8i + 7 of this k; the even lane
+        // stores the slot for even k, the odd lane for odd k
+        const unsigned lo = pack_bf16x2(h[k][0], h[k][1]), hi = pack_bf16x2(h[k][2], h[k][3]);
+        const unsigned plo = swap_adj(lo), phi = swap_adj(hi);
+        if ((c.lane & 1) == (k & 1))
+          *reinterpret_cast<u32x4*>(p.ws + c.xb + K::X_XN + n * (TP * D * 2) + frag_off(32, t, d & ~7)) =
+              (c.lane & 1) ? u32x4{plo, phi, lo, hi} : u32x4{lo, hi, plo, phi};
+      }
+    } else {
+#pragma unroll 1
+      for (int a0 = 0; a0 < AD; a0 += 4) {
+        f32x4 wv[4][4];
+#pragma unroll
+        for (int a = 0; a < 4; a++)
+#pragma unroll
+          for (int k = 0; k < 4; k++)
+            wv[a][k] = *reinterpret_cast<const f32x4*>(p.w_aout + (a0 + a) * D + 4 * c.lane + 256 * k);
+#pragma unroll
+        for (int a = 0; a < 4; a++) {
+          float s = 0.f;
+#pragma unroll
+          for (int k = 0; k < 4; k++)
+            s += wv[a][k][0] * h[k][0] + wv[a][k][1] * h[k][1] + wv[a][k][2] * h[k][2] + wv[a][k][3] * h[k][3];
+          s = wave_sum(s);
+          if (c.lane == 0) xt[a0 + a] += dt * (s + p.b_aout[a0 + a]);
+        }
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------- QKV
+template <class K>
+__device__ __forceinline__ void stage_qkv(const Params& p, const Ctx& c, int li, int l, int pg0, bool last) {
+  constexpr int R = K::RQ;
+  const int t = 16 * c.wave + c.lr;
+  if (16 * c.wave >= p.Tv) {
+    page_release<K>(c, pg0 + K::PQ);
+    return;
+  }
+  const bool tv = t < p.Tv;
+  wait_norm_rows(c);
+  f32x4 acc[K::NB][R];
+  uint32_t xo[K::NB];
+  tok_off<K>(p, c, K::X_XN, 32, 0, xo);
+  gemm<K, R, K::KX>(acc, c, pg0, xo);
+#pragma unroll
+  for (int rt = 0; rt < R; rt++) {
+    const int vr0 = 16 * (R * c.r + rt);  // wave-uniform: the tile lies within q, k or v
+    if (vr0 >= 256 * K::HX + 256) {       // v dims d..d+3 of token t, transposed
+      const int d = vr0 - (256 * K::HX + 256) + 4 * c.lq;
+#pragma unroll
+      for (int n = 0; n < K::NB; n++) {
+        if (!tv || n >= c.ns) continue;
+        unsigned short* vs = reinterpret_cast<unsigned short*>(p.ws + c.xb + K::X_VS) + ((li & 1) * K::NB + n) * TP * HD;
+        unsigned short* vr =
+            reinterpret_cast<unsigned short*>(p.vtcache) +
+            (((size_t)(c.grp + n * K::NGRP) * p.NL + l) * HD + d) * p.Lmax + p.Lp + t;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const unsigned short u = bf16_bits(acc[n][rt][i]);
+          vs[(d + i) * TP + t] = u;
+          if (last && c.j == l % K::G) vr[(size_t)i * p.Lmax] = u;
+        }
+      }
+      continue;
+    }
+    const int p0 = (vr0 < 256 * K::HX ? vr0 & 255 : vr0 - 256 * K::HX) / 2 + 2 * c.lq;  // first of two RoPE pairs
+    const uint32_t ro = tv ? (uint32_t)(t * 128 + p0) * 4 : OOB;
+    const u32x2 cs = ldb64<kCpPlain>(c.rc, ro), sn = ldb64<kCpPlain>(c.rs, ro);
+    const float c0 = as_f32(cs[0]), c1 = as_f32(cs[1]), s0 = as_f32(sn[0]), s1 = as_f32(sn[1]);
+#pragma unroll
+    for (int n = 0; n < K::NB; n++) {
+      const f32x4 v = acc[n][rt];
+      const unsigned plo = pack_bf16x2(v[0] * c0 - v[1] * s0, v[2] * c1 - v[3] * s1);
+      const unsigned phi = pack_bf16x2(v[1] * c0 + v[0] * s0, v[3] * c1 + v[2] * s1);
+      if (!tv || n >= c.ns) continue;
+      if (vr0 < 256 * K::HX) {
+        unsigned char* q = p.ws + c.xb + K::X_Q + (uint32_t)((n * K::HX + (vr0 >> 8)) * TP * HD * 2);
+        *reinterpret_cast<unsigned*>(q + frag_off(8, t, p0)) = plo;
+        *reinterpret_cast<unsigned*>(q + frag_off(8, t, p0 + 128)) = phi;
+      } else {
+        unsigned char* k = p.ws + c.xb + K::X_KS + (uint32_t)(((((li & 1) * K::NB + n) * TP + t) * HD + p0) * 2);
+        *reinterpret_cast<unsigned*>(k) = plo;
+        *reinterpret_cast<unsigned*>(k + 256) = phi;
+        if (last && c.j == l % K::G) {  // the caller's caches keep the last step's rows
+          bf16* kr = p.kcache + (((size_t)(c.grp + n * K::NGRP) * p.NL + l) * p.Lmax + p.Lp + t) * HD + p0;
+          *reinterpret_cast<unsigned*>(kr) = plo;
+          *reinterpret_cast<unsigned*>(kr + 128) = phi;
+        }
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------- attention
+// Item of rank r: slot an, head ah, prefix keys [kbeg, kend) in segments of up to SEGU 64-key units from
+// the ring (a segment's K pages, then its V^T pages), after this step's keys [sbeg, sbeg + nsfx) of the
+// XCD's copies, whose loads arrive with q. Wave w: query rows of tokens 16w..16w+15. Per segment: S^T = K Q^T of all
+// its keys, one softmax (rescaling what earlier segments left), O^T += V^T P^T of all its keys: the two
+// MFMA phases are free of the softmax's serial chain, which a loop over 32-key blocks paid per block
+// (ATT 25 us per layer at 16 samples, 14 at 8).
+// K rows are permuted inside each 32-key block: row 4a + i of tile kt is key 8a + 4kt + i, so a lane's S^T
+// values of tiles (0, 1) are keys 8 lq .. 8 lq + 7, the P^T operand, and V^T fragments are read whole.
+template <class K>
+__device__ __forceinline__ void stage_att(const Params& p, const Ctx& c, int li, int pgk) {
+  constexpr int NT = 4 * K::SEGU;  // key tiles of a segment
+  if (16 * c.wave >= p.Tv || c.an >= c.ns) {
+    page_release<K>(c, pgk + 4 * c.nun);
+    return;
+  }
+  const int t = 16 * c.wave + c.lr;
+  const bool tv = t < p.Tv;
+  const float qscale = 1.4426950408889634f / 16.0f;  // log2(e) / sqrt(256)
+  const uint32_t pbase = (uint32_t)(c.r * TP + t);
+  if (c.nun == 0 && c.nsfx <= 0) {  // empty chunk: weight 0 in the combine
+    if (tv && c.lq == 0) *reinterpret_cast<f32x2*>(p.ws + c.xb + K::X_ML + pbase * 8) = f32x2{-1e30f, 0.f};
+    return;
+  }
+  u32x4 qf[8], skf[2][8], sv[16];
+  {
+    const uint32_t qb = tv ? c.xb + K::X_Q + (uint32_t)((c.an * K::HX + c.ah) * TP * HD * 2) + frag_off(8, t, 8 * c.lq) : OOB;
+#pragma unroll
+    for (int ks = 0; ks < 8; ks++) qf[ks] = ldb128<kCpSc1>(c.ws, qb + ks * 1024);
+    // this step's keys (rows past nsfx: zeros) and the 16-byte groups of their V^T that start below nsfx
+    const uint32_t kb = c.xb + K::X_KS + (uint32_t)((((li & 1) * K::NB + c.an) * TP + c.sbeg) * HD * 2);
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++) {
+      const int key = 8 * (c.lr >> 2) + 4 * kt + (c.lr & 3);
+      const uint32_t a = key < c.nsfx ? kb + key * (HD * 2) + c.lq * 16 : OOB;
+#pragma unroll
+      for (int ks = 0; ks < 8; ks++) skf[kt][ks] = ldb128<kCpSc1>(c.ws, a + ks * 64);
+    }
+    const uint32_t vb = c.xb + K::X_VS + (uint32_t)((((li & 1) * K::NB + c.an) * TP * HD + c.lr * TP + c.sbeg + 8 * c.lq) * 2);
+    const uint32_t va = 8 * c.lq < c.nsfx ? vb : OOB;
+#pragma unroll
+    for (int dt = 0; dt < 16; dt++) sv[dt] = ldb128<kCpSc1>(c.ws, va + dt * (16 * TP * 2));
+  }
+  // S^T of one key tile
+  auto score = [&](const u32x4 (&kf)[8]) __attribute__((always_inline)) {
+    f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 8; ks += 2) {
+      a = mfma16(kf[ks], qf[ks], a);
+      b = mfma16(kf[ks + 1], qf[ks + 1], b);
+    }
+    return a + b;
+  };
+  // keys 8 lq + 4 kt + i >= nv of a 32-key block: S = -inf, V = 0
+  auto smask = [&](f32x4& s, int kt, int nv) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      if (8 * c.lq + 4 * kt + i >= nv) s[i] = -1e30f;
+  };
+  auto vmask = [&](u32x4& v, int nv) __attribute__((always_inline)) {
+    const int q = min(max(nv - 8 * c.lq, 0), 8);
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] &= q >= 2 * e + 2 ? 0xffffffffu : (q == 2 * e + 1 ? 0xffffu : 0u);
+  };
+  auto pack_p = [&](const f32x4& a, const f32x4& b) __attribute__((always_inline)) {
+    return u32x4{pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]), pack_bf16x2(b[0], b[1]), pack_bf16x2(b[2], b[3])};
+  };
+  float m = -1e30f, lsum = 0.f;
+  f32x4 o[16];
+  // softmax of N key tiles (pairs = 32-key blocks) against the running (m, l) -> P^T operands; returns the
+  // factor of what came before
+  auto softmax = [&](auto& x, auto& pb) __attribute__((always_inline)) {
+    constexpr int N = sizeof(x) / sizeof(f32x4);
+    float bm = -1e30f;
+#pragma unroll
+    for (int q = 0; q < N; q++) bm = fmaxf(bm, fmaxf(fmaxf(x[q][0], x[q][1]), fmaxf(x[q][2], x[q][3])));
+    const float mnew = fmaxf(m, cols_max(bm) * qscale);
+    const float alpha = exp2_w(m - mnew);
+    m = mnew;
+    float ps = 0.f;
+#pragma unroll
+    for (int q = 0; q < N; q += 2) {
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          x[q + h][i] = exp2_w(fmaf(x[q + h][i], qscale, -m));
+          ps += x[q + h][i];
+        }
+      pb[q / 2] = pack_p(x[q], x[q + 1]);
+    }
+    lsum = lsum * alpha + cols_sum(ps);
+    return alpha;
+  };
+  {
+    f32x4 s[2];
+    u32x4 pb[1];
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++) {
+      s[kt] = score(skf[kt]);
+      smask(s[kt], kt, c.nsfx);
+    }
+    if (c.nsfx > 0) softmax(s, pb);
+    else pb[0] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int dt = 0; dt < 16; dt++) {
+      vmask(sv[dt], c.nsfx);
+      o[dt] = mfma16(sv[dt], pb[0], f32x4{0.f, 0.f, 0.f, 0.f});
+    }
+  }
+#pragma unroll 1
+  for (int u0 = 0; u0 < c.nun; u0 += K::SEGU) {
+    const int nu = min(K::SEGU, c.nun - u0);       // units of this segment
+    const int nv0 = c.kend - (c.kbeg + 64 * u0);    // its valid keys
+    const int pk = pgk + 4 * u0, pv = pk + 2 * nu;  // its K and V^T pages
+    f32x4 s[NT];
+#pragma unroll
+    for (int u = 0; u < K::SEGU; u++) {
+#pragma unroll
+      for (int q = 0; q < 4; q++) s[4 * u + q] = f32x4{-1e30f, -1e30f, -1e30f, -1e30f};
+      if (u >= nu) continue;
+      page_wait<K>(c, pk + 2 * u + 1);
+      u32x4 kf[2][8];
+      auto rd = [&](int q) {
+        const uint32_t a = ((pk + 2 * u + (q >> 1)) % RING) * PAGE + c.lane * 16 + (q & 1) * 8192;
+#pragma unroll
+        for (int ks = 0; ks < 8; ks++) kf[q & 1][ks] = *reinterpret_cast<const u32x4*>(fg_lds + a + ks * 1024);
+      };
+      rd(0);
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        if (q + 1 < 4) rd(q + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        s[4 * u + q] = score(kf[q & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      page_release<K>(c, pk + 2 * u + 2);
+      if (u == nu - 1 && nv0 < 64 * nu) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) smask(s[4 * u + q], q & 1, nv0 - 64 * u - 32 * (q >> 1));
+      }
+    }
+    u32x4 pb[NT / 2];
+    const float alpha = softmax(s, pb);
+#pragma unroll
+    for (int dt = 0; dt < 16; dt++) o[dt] *= alpha;
+#pragma unroll
+    for (int u = 0; u < K::SEGU; u++) {
+      if (u >= nu) continue;
+      page_wait<K>(c, pv + 2 * u + 1);
+      u32x4 vf[2][8];
+      auto rd = [&](int q) {  // half q & 1 of the dims of block q / 2
+        const uint32_t a = ((pv + 2 * u + (q >> 1)) % RING) * PAGE + c.lane * 16 + (q & 1) * 8192;
+#pragma unroll
+        for (int d8 = 0; d8 < 8; d8++) vf[q & 1][d8] = *reinterpret_cast<const u32x4*>(fg_lds + a + d8 * 1024);
+      };
+      const bool part = u == nu - 1 && nv0 < 64 * nu;
+      rd(0);
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        if (q + 1 < 4) rd(q + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (part) {
+#pragma unroll
+          for (int d8 = 0; d8 < 8; d8++) vmask(vf[q & 1][d8], nv0 - 64 * u - 32 * (q >> 1));
+        }
+#pragma unroll
+        for (int d8 = 0; d8 < 8; d8++)
+          o[8 * (q & 1) + d8] = mfma16(vf[q & 1][d8], pb[2 * u + (q >> 1)], o[8 * (q & 1) + d8]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      page_release<K>(c, pv + 2 * u + 2);
+    }
+  }
+  // O^T / l in the O projection's operand order, whole 16-byte slots (see pi05_bs1.hip)
+  const float inv = lsum > 0.f ? 1.0f / lsum : 0.f;
+  const bool odd = c.lq & 1;
+  const uint32_t ob = c.xb + K::X_ATTP + (uint32_t)((c.r * 4 + c.wave) * 8192 + (c.lr * 4 + (c.lq >> 1) + 2 * (c.lq & 1)) * 16);
+#pragma unroll
+  for (int ks = 0; ks < 8; ks++) {
+    const unsigned a0 = pack_bf16x2(o[2 * ks][0] * inv, o[2 * ks][1] * inv);
+    const unsigned a1 = pack_bf16x2(o[2 * ks][2] * inv, o[2 * ks][3] * inv);
+    const unsigned b0 = pack_bf16x2(o[2 * ks + 1][0] * inv, o[2 * ks + 1][1] * inv);
+    const unsigned b1 = pack_bf16x2(o[2 * ks + 1][2] * inv, o[2 * ks + 1][3] * inv);
+    const LanePair s0 = swap16(a0, b0), s1 = swap16(a1, b1);
+    if (tv)  // rows past Tv are never read
+      *reinterpret_cast<u32x4*>(p.ws + ob + ks * 1024) = odd ? u32x4{s0.lo, s1.lo, b0, b1} : u32x4{a0, a1, s0.hi, s1.hi};
+  }
+  if (tv && c.lq == 0) *reinterpret_cast<f32x2*>(p.ws + c.xb + K::X_ML + pbase * 8) = f32x2{m, lsum};
+}
+
+// ---------------------------------------------------------------- combine
+// Fragment id = (slot, head, k-step) of token tile w: wave w of rank r takes ids FPR r .. + FPR - 1 (with
+// G = 4: id r of ranks < 16). A lane owns one 16-byte slot (token 16 w + lane / 4, 8 dims).
+template <class K>
+__device__ __forceinline__ void stage_comb(const Params& p, const Ctx& c) {
+  constexpr int NF = K::FPR > 0 ? K::FPR : 1;
+  const int id0 = c.r * NF;
+  if (16 * c.wave >= p.Tv || id0 >= K::NB * K::HX * 8) return;
+  const int nh = id0 >> 3, n = nh / K::HX;  // a rank's ids share their (slot, head)
+  if (n >= c.ns) return;
+  xcd_wait(c, (K::NKC == 32 ? 0xffffffffu : ((1u << (K::NKC & 31)) - 1u)) << (nh * K::NKC));
+  const int t = 16 * c.wave + (c.lane >> 2);
+  const bool tv = t < p.Tv;
+  u32x2 ml[K::NKC];
+  u32x4 v[NF][K::NKC];
+#pragma unroll
+  for (int k = 0; k < K::NKC; k++) {
+    const int rr = nh * K::NKC + k;
+    ml[k] = ldb64<kCpSc1>(c.ws, tv ? c.xb + K::X_ML + (uint32_t)(rr * TP + t) * 8 : OOB);
+#pragma unroll
+    for (int f = 0; f < NF; f++)
+      v[f][k] = ldb128<kCpSc1>(c.ws, tv ? c.xb + K::X_ATTP + (uint32_t)((rr * 4 + c.wave) * 8192 + ((id0 + f) & 7) * 1024 + c.lane * 16) : OOB);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  float M = -1e30f;
+#pragma unroll
+  for (int k = 0; k < K::NKC; k++) M = fmaxf(M, as_f32(ml[k][0]));
+  float wt[K::NKC], L = 0.f;
+#pragma unroll
+  for (int k = 0; k < K::NKC; k++) {
+    wt[k] = as_f32(ml[k][1]) * exp2_w(as_f32(ml[k][0]) - M);
+    L += wt[k];
+  }
+  const float inv = L > 0.f ? 1.0f / L : 0.f;
+#pragma unroll
+  for (int f = 0; f < NF; f++) {
+    float u[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) u[e] = 0.f;
+#pragma unroll
+    for (int k = 0; k < K::NKC; k++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const unsigned d = wt[k] != 0.f ? v[f][k][e] : 0u;  // empty chunks hold no partial
+        u[2 * e] = fmaf(wt[k], bf_lo(d), u[2 * e]);
+        u[2 * e + 1] = fmaf(wt[k], bf_hi(d), u[2 * e + 1]);
+      }
+    u32x4 out;
+#pragma unroll
+    for (int e = 0; e < 4; e++) out[e] = pack_bf16x2(u[2 * e] * inv, u[2 * e + 1] * inv);
+    const int ks = (nh % K::HX) * 8 + ((id0 + f) & 7);
+    *reinterpret_cast<u32x4*>(p.ws + c.xb + K::X_ATTN + (uint32_t)(((n * 4 + c.wave) * 8 * K::HX + ks) * 1024 + c.lane * 16)) = out;
+  }
+}
+
+// Stores the fp32 partial sums of the rank's rows (row group rg, window index wd of the group).
+template <class K>
+__device__ __forceinline__ void store_part(const Params& p, const Ctx& c, uint32_t part, int wd, int rg,
+                                           const f32x4 (&acc)[K::NB][K::RP]) {
+  const int t = 16 * c.wave + c.lr;
+  if (t >= p.Tv) return;
+#pragma unroll
+  for (int n = 0; n < K::NB; n++) {
+    if (n >= c.ns) continue;
+#pragma unroll
+    for (int rt = 0; rt < K::RP; rt++)
+      stb128<kCpPart<K>>(c.ws, c.part + part + wd * (K::PB1 / 4) +
+                                  (uint32_t)(((n * TP + t) * D + 16 * (K::RP * rg + rt) + 4 * c.lq) * 4),
+                         as_u32x4(acc[n][rt]));
+  }
+}
+
+// Ranks whose combine wrote K window `win` (heads 2 win, 2 win + 1) of the attention output.
+template <class K>
+__device__ __forceinline__ uint32_t comb_ranks(int win) {
+  if constexpr (K::FPR == 0) return 0xffffu;
+  constexpr int NF = K::FPR > 0 ? K::FPR : 1, W = 16 / NF;  // ranks per window and slot
+  uint32_t m = 0;
+#pragma unroll
+  for (int n = 0; n < K::NB; n++) m |= ((W >= 32 ? 0u : 1u << W) - 1u) << ((n * K::HX * 8 + 16 * win) / NF);
+  return m;
+}
+
+template <class K>
+__device__ __forceinline__ void stage_oproj(const Params& p, const Ctx& c, int pg0) {
+  if (16 * c.wave >= p.Tv) {
+    page_release<K>(c, pg0 + K::PO);
+    return;
+  }
+  const int win = c.r / (NR / K::C), rg = c.r % (NR / K::C);
+  xcd_wait(c, comb_ranks<K>(win));
+  f32x4 acc[K::NB][K::RP];
+  uint32_t xo[K::NB];
+  tok_off<K>(p, c, K::X_ATTN, 8 * K::HX, 16 * win, xo);
+  gemm<K, K::RP, K::KO>(acc, c, pg0, xo);
+  store_part<K>(p, c, 0, K::C * c.j + win, rg, acc);
+}
+
+template <class K>
+__device__ __forceinline__ void stage_gu(const Params& p, const Ctx& c, int pg0) {
+  if (16 * c.wave >= p.Tv) {
+    page_release<K>(c, pg0 + K::PGU);
+    return;
+  }
+  wait_norm_rows(c);
+  uint32_t xo[K::NB];
+  tok_off<K>(p, c, K::X_XN, 32, 0, xo);
+#pragma unroll 1
+  for (int q = 0; q < K::PG; q++) {
+    f32x4 acc[K::NB][K::RGP];
+    // operand offsets are derived in each pass (hoisted out of the loop they spilled)
+#pragma unroll
+    for (int n = 0; n < K::NB; n++) asm volatile("" : "+v"(xo[n]));
+    gemm<K, K::RGP, K::KX>(acc, c, pg0 + q * (K::PGU / K::PG), xo);
+    int t = 16 * c.wave + c.lr;
+    asm volatile("" : "+v"(t));  // the store addresses are derived here, not kept live over the GEMM
+    if (t >= p.Tv) continue;
+    // rows 2f, 2f + 1 = gate f, up f: the lane's columns f = 8 (row tile) + 2 lq + (0, 1) of the rank's slice.
+    // One exchange with lane ^ 16 per pair of row tiles gives a lane 4 consecutive columns (8 bytes).
+#pragma unroll
+    for (int n = 0; n < K::NB; n++) {
+      if (n >= c.ns) continue;
+#pragma unroll
+      for (int rt = 0; rt < K::RGP; rt += 2) {
+        const f32x4 a = acc[n][rt], b = acc[n][rt + 1];
+        const unsigned p0 = pack_bf16x2(gelu_tanh(a[0]) * a[1], gelu_tanh(a[2]) * a[3]);
+        const unsigned p1 = pack_bf16x2(gelu_tanh(b[0]) * b[1], gelu_tanh(b[2]) * b[3]);
+        const bool odd = c.lq & 1;
+        const LanePair sw = swap16(p0, p1);
+        const unsigned recv = odd ? sw.lo : sw.hi;
+        const int f = 8 * (K::RG * c.r + K::RGP * q + rt) + (odd ? 8 + 2 * (c.lq - 1) : 2 * c.lq);
+        *reinterpret_cast<u32x2*>(p.ws + c.xb + K::X_H + n * (TP * (FF / K::G) * 2) + frag_off(128 / K::G, t, f)) =
+            odd ? u32x2{recv, p1} : u32x2{p0, recv};
+      }
+    }
+  }
+}
+
+template <class K>
+__device__ __forceinline__ void stage_dn(const Params& p, const Ctx& c, int pg0) {
+  if (16 * c.wave >= p.Tv) {
+    page_release<K>(c, pg0 + K::PD);
+    return;
+  }
+  const int win = c.r / (NR / K::C), rg = c.r % (NR / K::C);
+  constexpr int GW = 8 * K::G;  // gate/up ranks per 1024-column window
+  xcd_wait(c, GW == 32 ? 0xffffffffu : ((1u << (GW & 31)) - 1u) << (GW * win));
+  f32x4 acc[K::NB][K::RP];
+  uint32_t xo[K::NB];
+  tok_off<K>(p, c, K::X_H, 128 / K::G, 32 * win, xo);
+  gemm<K, K::RP, K::KD>(acc, c, pg0, xo);
+  store_part<K>(p, c, K::PB - K::PB1, K::C * c.j + win, rg, acc);
+}
+
+// ---------------------------------------------------------------- instrumentation
+__device__ __forceinline__ void mark(const Params& p, const Ctx& c, int idx, uint64_t& t0) {
+  if (p.stage_cycles && blockIdx.x == 0 && c.wave == 0 && c.lane == 0) {
+    const uint64_t now = __builtin_amdgcn_s_memrealtime();
+    p.stage_cycles[idx] += now - t0;  // 0-7 stages N1 QKV ATT COMB O N2 GU DN, 8 final, 9 XCD barrier and signals
+    t0 = now;
+  }
+}
+
+// ---------------------------------------------------------------- kernel
+template <int G, int NB>
+__global__ void __launch_bounds__(NTH, 1) pi05_group_kernel(Params p) {
+  using K = Cfg<G, NB>;
+  Ctx c;
+  const int tid = threadIdx.x;
+  c.x = blockIdx.x & 7;
+  c.grp = c.x / G;
+  c.j = c.x % G;
+  c.ns = min(NB, (p.B - c.grp + K::NGRP - 1) / K::NGRP);
+  if (p.B <= c.grp) return;  // no sample for this group: the whole workgroup
+  c.lane = tid & 63;
+  c.wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  c.lr = c.lane & 15;
+  c.lq = c.lane >> 4;
+  c.r = blockIdx.x >> 3;
+  c.ws = make_rsrc(p.ws, K::WS);
+  c.rc = make_rsrc(p.rope_cos, (uint32_t)(p.Tv * 128 * 4));
+  c.rs = make_rsrc(p.rope_sin, (uint32_t)(p.Tv * 128 * 4));
+  c.xb = K::OFF_XCD + (uint32_t)c.x * K::XB;
+  c.part = K::OFF_PART + (uint32_t)c.grp * K::PB;
+  c.lds_addr = (uint32_t)(uintptr_t)fg_lds;
+  c.err = reinterpret_cast<unsigned*>(p.ws + OFF_CTRL + 8);
+  {
+    c.an = c.r / (K::HX * K::NKC);
+    c.ah = (c.r / K::NKC) % K::HX;
+    const int kc = c.r % K::NKC, chunk = 64 * ((p.Lp + 64 * K::NKC - 1) / (64 * K::NKC));
+    c.kbeg = min(kc * chunk, p.Lp);
+    c.kend = min(c.kbeg + chunk, p.Lp);
+    c.nun = c.an < c.ns ? (c.kend - c.kbeg + 63) / 64 : 0;
+    c.sbeg = kc * K::SK;
+    c.nsfx = min(p.Tv - c.sbeg, K::SK);
+  }
+  if (tid < 16) ctl_st<K>(tid, 0u);
+  if (tid == 0 && xcc_id() != (unsigned)c.x) atomicOr(c.err, kErrXcd);
+  const uint64_t seq = ld_flag(reinterpret_cast<const uint64_t*>(p.ws + OFF_CTRL));
+  __syncthreads();  // the only workgroup barrier: LDS control words are initialised
+  if (c.wave >= NCW) {
+    Loader<K> L{p, c, c.wave - NCW};
+    L.run();
+    return;
+  }
+  c.e = c.eg = seq << 32;
+  const int NL = p.NL;
+  const int t = c.r + 32 * (c.wave >> 1);
+  const bool nw = (c.wave & 1) == (c.r >> 4) && t < p.Tv;  // this wave owns a token in the norm stages
+  if (nw && c.lane < AD)
+    for (int n = 0; n < c.ns; n++)
+      reinterpret_cast<float*>(fg_lds + K::L_XT)[(2 * n + (c.wave >> 1)) * AD + c.lane] =
+          p.x_t[((size_t)(c.grp + n * K::NGRP) * p.xt_rows + t) * AD + c.lane];
+  const float dt = -1.0f / (float)p.S;
+  const int ppl = K::PQ + 4 * c.nun + K::PO + K::PGU + K::PD;
+  int pb = 0;  // first ring page of the layer
+  uint64_t t0 = __builtin_amdgcn_s_memrealtime();
+#pragma unroll 1
+  for (int step = 0; step < p.S; step++) {
+#pragma unroll 1
+    for (int l = 0; l < NL; l++, pb += ppl) {
+      launder(c);
+      const int li = step * NL + l;
+      const float* mod_in = p.mods + ((size_t)li * 2 + 0) * 3 * D;
+      const float* mod_post = p.mods + ((size_t)li * 2 + 1) * 3 * D;
+      if (nw) {
+        if (l == 0)
+          stage_norm<K, 0>(p, c, 0, nullptr, mod_in, mod_in + D, 0.f);
+        else
+          stage_norm<K, 1>(p, c, K::PB - K::PB1, mod_post - 6 * D + 2 * D, mod_in, mod_in + D, 0.f);
+      }
+      mark(p, c, 0, t0);
+      xcd_signal(p, c);
+      launder(c);
+      mark(p, c, 9, t0);
+      stage_qkv<K>(p, c, li, l, pb, step == p.S - 1);
+      mark(p, c, 1, t0);
+      xcd_sync(p, c);
+      launder(c);
+      mark(p, c, 9, t0);
+      stage_att<K>(p, c, li, pb + K::PQ);
+      mark(p, c, 2, t0);
+      xcd_signal(p, c);
+      launder(c);
+      mark(p, c, 9, t0);
+      stage_comb<K>(p, c);
+      mark(p, c, 3, t0);
+      xcd_signal(p, c);
+      launder(c);
+      mark(p, c, 9, t0);
+      stage_oproj<K>(p, c, pb + K::PQ + 4 * c.nun);
+      mark(p, c, 4, t0);
+      part_signal<K>(p, c);
+      launder(c);
+      mark(p, c, 9, t0);
+      if (nw) stage_norm<K, 1>(p, c, 0, mod_in + 2 * D, mod_post, mod_post + D, 0.f);
+      mark(p, c, 5, t0);
+      xcd_signal(p, c);
+      launder(c);
+      mark(p, c, 9, t0);
+      stage_gu<K>(p, c, pb + K::PQ + 4 * c.nun + K::PO);
+      mark(p, c, 6, t0);
+      xcd_signal(p, c);
+      launder(c);
+      mark(p, c, 9, t0);
+      stage_dn<K>(p, c, pb + K::PQ + 4 * c.nun + K::PO + K::PGU);
+      mark(p, c, 7, t0);
+      part_signal<K>(p, c);
+    }
+    if (nw) {
+      const int li = step * NL + NL - 1;
+      const float* gl = p.mods + ((size_t)li * 2 + 1) * 3 * D + 2 * D;
+      const float* mf = p.mod_final + (size_t)step * 3 * D;
+      stage_norm<K, 2>(p, c, K::PB - K::PB1, gl, mf, mf + D, dt);
+    }
+    mark(p, c, 8, t0);
+  }
+  if (c.j == 0 && nw && c.lane < AD)
+    for (int n = 0; n < c.ns; n++)
+      p.x_t[((size_t)(c.grp + n * K::NGRP) * p.xt_rows + t) * AD + c.lane] =
+          reinterpret_cast<float*>(fg_lds + K::L_XT)[(2 * n + (c.wave >> 1)) * AD + c.lane];
+  // The launch sequence advances when the last group is done: the groups do not wait for one another, and
+  // a workgroup that starts late must still read this launch's number. (This wave has seen every wave of
+  // its group past the prologue.)
+  if (c.j == 0 && c.r == 0 && c.wave == 0 && c.lane == 0) {
+    unsigned* done = reinterpret_cast<unsigned*>(p.ws + OFF_DONE);
+    const unsigned groups = (unsigned)min(p.B, K::NGRP);
+    if (__hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == groups - 1) {
+      __hip_atomic_store(done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(reinterpret_cast<unsigned*>(p.ws + kWsOwner), kOwnerPi05Group, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(reinterpret_cast<uint64_t*>(p.ws + OFF_CTRL), seq + 1, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+}
+
+struct Choice {
+  const void* kernel;
+  unsigned lds;
+  size_t ws;
+};
+template <int G, int NB>
+Choice choice() {
+  return {(const void*)pi05_group_kernel<G, NB>, Cfg<G, NB>::LDS, Cfg<G, NB>::WS};
+}
+// Wider groups stream fewer weights per XCD but exchange partial sums between XCDs. Two samples per group
+// share every weight fragment. ms per launch (Lp = 968, Tv = 50, 10 steps), against the stage engine's:
+//   batch 2   (4, 1) 6.2, (4, 2) 7.1               stage engine 16.7
+//   batch 4   (4, 2) 8.4, (2, 1) 8.4 (Tv = 10: 6.0 against 6.4)      17.0
+//   batch 8   (2, 2) 11.2, (1, 1) 12.8                               17.4
+//   batch 16  (1, 2) 16.9, (2, 4) 17.6                               18.9
+// Past 16 samples an XCD would hold more than two, whose tokens fill the stage engine's tiles.
+Choice pick(int batch) {
+  if (batch <= 2) return choice<4, 1>();
+  if (batch <= 4) return choice<4, 2>();
+  if (batch <= 8) return choice<2, 2>();
+  return choice<1, 2>();
+}
+
+}  // namespace pg
+
+// ---------------------------------------------------------------- host
+bool pi05_group_eligible(int batch, int Tv) { return batch >= 2 && batch <= 16 && Tv >= 1 && Tv <= pg::TP; }
+size_t pi05_group_workspace_bytes(int batch) { return pg::pick(batch).ws; }
+
+int pi05_denoise_group(const fa_pi05_args* a, fa_stream_t stream) {
+  using namespace fa::pg;
+  const Choice k = pick(a->batch);
+  int rc = host::check_device(k.kernel, NTH, k.lds, NWG, "fa_pi05_denoise");
+  if (rc != FA_OK) return rc;
+  Params p;
+  p.w1 = static_cast<const bf16*>(a->w1);
+  p.wo = static_cast<const bf16*>(a->wo);
+  p.w2 = static_cast<const bf16*>(a->w2);
+  p.w3 = static_cast<const bf16*>(a->w3);
+  p.mods = a->mods;
+  p.mod_final = a->mod_final;
+  p.rope_cos = a->rope_cos;
+  p.rope_sin = a->rope_sin;
+  p.w_ain = a->w_ain;
+  p.b_ain = a->b_ain;
+  p.w_aout = a->w_aout;
+  p.b_aout = a->b_aout;
+  p.kcache = static_cast<bf16*>(a->kcache);
+  p.vtcache = static_cast<bf16*>(a->vtcache);
+  p.x_t = a->x_t;
+  p.stage_cycles = a->stage_cycles;
+  p.ws = static_cast<unsigned char*>(a->workspace);
+  p.NL = a->num_layers;
+  p.Lp = a->Lp;
+  p.Lmax = a->Lmax;
+  p.S = a->num_steps;
+  p.Tv = a->Tv;
+  p.B = a->batch;
+  p.xt_rows = a->xt_rows;
+  if (a->srows > 0 && (rc = pi05_kv_handoff(a, stream)) != FA_OK) return rc;
+  void* args[] = {&p};
+  return host::coop_launch(k.kernel, NWG, NTH, args, k.lds, stream, "fa_pi05_denoise (batched)");
+}
+
+}  // namespace fa

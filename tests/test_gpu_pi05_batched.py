@@ -40,6 +40,37 @@ def test_batched_edge_shapes(gpu, B, Lp, Tv, S):
     _check(P.make_case(NL=2, Lp=Lp, Tv=Tv, S=S, batch=B, seed=B + Lp + Tv), gpu)
 
 
+# Every group shape (batch 2, 3-4, 5-8, 9-16: one or two samples on one, two or four XCDs; odd batches leave
+# a group with one sample or none) and the stage engine past them (17), at one and four token tiles,
+# prefixes that end on, before and after a 64-key unit of the attention, and prefixes long enough
+# (Lp > 1024) for a second segment of units per key chunk.
+@pytest.mark.parametrize("B,Lp,Tv,S,NL", [(2, 64, 1, 2, 1), (2, 1030, 64, 1, 1), (3, 65, 16, 2, 2), (4, 1200, 33, 1, 1),
+                                         (5, 63, 64, 1, 1), (8, 1025, 17, 1, 2), (9, 0, 49, 1, 1), (16, 129, 10, 2, 1),
+                                         (17, 70, 9, 1, 1)])
+def test_batched_group_shapes(gpu, B, Lp, Tv, S, NL):
+    _check(P.make_case(NL=NL, Lp=Lp, Tv=Tv, S=S, batch=B, seed=B + Lp + Tv), gpu)
+
+
+def test_batched_repeats_on_one_workspace(gpu):
+    """Launches of different group shapes, of the batch-1 kernel and of the stage engine (a workspace too
+    small for the groups) on one workspace, each against its first result."""
+    cs = [P.make_case(NL=1, Lp=90, Tv=20, S=2, batch=B, seed=B) for B in (2, 4, 8, 16)]
+    n = max(pi05.workspace(gpu, c["batch"], 20, 112).numel() for c in cs)
+    raw = torch.zeros(n + 256, dtype=torch.uint8, device=gpu)
+    ws = raw[(-raw.data_ptr()) % 256:][:n]
+    first = {}
+    for r in range(2):
+        for c in cs:
+            out = P.run_gpu_batched(c, gpu, ws=ws)[0]
+            assert pi05.read_status(ws) == 0
+            assert np.array_equal(out, first.setdefault(c["batch"], out))
+        one = P.run_gpu(P.make_case(NL=1, Lp=90, Tv=20, S=2, seed=2), gpu, ws=ws)[0]
+        assert np.abs(one - first.setdefault(1, one)).max() <= MAX_ABS  # the exchange parity moves its last bit
+    small = ws[:(8 << 20)]  # room for the stage engine at batch 2 only
+    out = P.run_gpu_batched(cs[0], gpu, ws=small)[0]
+    assert np.abs(out - first[2]).max() <= MAX_ABS
+
+
 def test_batched_baseline_config2(gpu):
     """The batch-16 benchmark workload vs the fp32 oracle: batch 16, 18 layers, Lp=968, Tv=50, 10 steps."""
     _check(P.make_case(NL=18, Lp=968, Tv=50, S=10, batch=16), gpu)
