@@ -59,7 +59,7 @@ constexpr uint32_t kWsMaxCounters = 1024;
 constexpr uint32_t kWsGroupFlags = 16384;  // [8 XCD][32 rank][4 wave] u64
 constexpr uint32_t kWsDataBase = 24576;
 constexpr unsigned kOwnerPi05Bs1 = 1, kOwnerPi05Batched = 2, kOwnerMa2Bs1 = 3, kOwnerMa2Generic = 4,
-                   kOwnerPrefill = 5, kOwnerPi05Group = 6;
+                   kOwnerPrefill = 5, kOwnerPi05Group = 6, kOwnerMa2Group = 7;
 
 __device__ __forceinline__ rsrc_t make_rsrc(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, kRsrcWord3);

@@ -63,4 +63,9 @@ bool ma2_bs1_eligible(int batch, int Tv, int Lkmax);
 size_t ma2_bs1_workspace_bytes();
 int ma2_bs1_launch(const fa_ma2_args* a, fa_stream_t stream);
 
+// MolmoAct2 batches of up to 16 samples on groups of XCDs (ma2_group.hip).
+bool ma2_group_eligible(int batch, int Tv);
+size_t ma2_group_workspace_bytes(int batch, int Tv);
+int ma2_group_launch(const fa_ma2_args* a, fa_stream_t stream);
+
 }  // namespace fa

@@ -21,6 +21,8 @@
 //          (large batches: a GATE stage applies the activation to the summed partials)
 //   DN     [M x 768] = m W_dn^T + b_dn
 // then the final norm, action projection and Euler update of x_t[:, :adim].
+#include <algorithm>
+
 #include "engine.h"
 #include "ma2_attn.h"
 #include "../../include/flashact_mi355x.h"
@@ -768,7 +770,8 @@ extern "C" size_t fa_ma2_workspace_bytes(int batch, int Tv, int Lkmax) {
   if (batch < 1 || Tv < 1 || Tv > ma2::MAX_TV || Lkmax < 16 || (size_t)batch * Tv > (size_t)ma2::MAX_TOKENS) return 0;
   if (ma2_bs1_eligible(batch, Tv, Lkmax)) return ma2_bs1_workspace_bytes();
   const size_t n = ma2::layout_for(batch, Tv, Lkmax).total;
-  return n < 0xffffffffull ? n : 0;
+  if (n >= 0xffffffffull) return 0;
+  return ma2_group_eligible(batch, Tv) ? std::max(n, ma2_group_workspace_bytes(batch, Tv)) : n;
 }
 
 extern "C" int fa_ma2_max_batch(void) { return ma2::MAX_TOKENS / ma2::MAX_TV; }
@@ -815,11 +818,17 @@ extern "C" int fa_ma2_flow(const fa_ma2_args* a, fa_stream_t stream) {
                       MAX_TOKENS);
   if ((size_t)a->batch * a->num_layers * a->Lkmax * D * 2 >= 0xffffffffull)
     return host::fail(FA_ERR_INVALID_ARG, "fa_ma2_flow: context caches exceed the 4 GB buffer range");
-  const size_t need = fa_ma2_workspace_bytes(a->batch, a->Tv, a->Lkmax);
+  const bool bs1 = ma2_bs1_eligible(a->batch, a->Tv, a->Lkmax);
+  const size_t whole = fa_ma2_workspace_bytes(a->batch, a->Tv, a->Lkmax);
+  const size_t need = bs1 || whole == 0 ? whole : layout_for(a->batch, a->Tv, a->Lkmax).total;
   if (need == 0 || a->workspace_bytes < need)
     return host::fail(FA_ERR_INVALID_ARG, "fa_ma2_flow: workspace_bytes=%zu < required %zu", a->workspace_bytes,
                       need);
-  if (ma2_bs1_eligible(a->batch, a->Tv, a->Lkmax)) return ma2_bs1_launch(a, stream);
+  if (bs1) return ma2_bs1_launch(a, stream);
+  // Up to 16 samples, groups of XCDs; past that (or in a workspace with no room for the groups) the
+  // stage engine.
+  if (ma2_group_eligible(a->batch, a->Tv) && a->workspace_bytes >= ma2_group_workspace_bytes(a->batch, a->Tv))
+    return ma2_group_launch(a, stream);
   const bool sm = small_cfg(a->batch * a->Tv);
   const void* kern = sm ? (const void*)ma2_kernel<1, 2, 2> : (const void*)ma2_kernel<3, 2, 4>;
   int rc = host::check_device(kern, NTHR, LDS_BYTES, NWG, "fa_ma2_flow");

@@ -27,24 +27,22 @@
 // feeds one XCD at 0.85-0.95 TB/s while all eight read (1.0 with four, 1.34 alone): 37 us per layer with
 // G = 1, 19 with G = 2, 10 with G = 4. The stage engine at these batches had 40 to 180 GEMM items for the 256
 // CUs in every stage but gate/up, and eight grid barriers of about 2 us per layer.
-#include "fa_device.h"
+#include "group.h"
 #include "../../include/flashact_mi355x.h"
 #include "fa_host.h"
 
 namespace fa {
 namespace pg {
+using namespace fa::grp;
 
 constexpr int D = 1024, HD = 256, AD = 32, FF = 4096, QD = 2048;
-constexpr int NX = 8, NR = 32, NWG = 256, TP = 64;
-constexpr int NCW = 4, NLW = 2, NTH = 64 * (NCW + NLW);  // compute waves, loader waves
-constexpr int RING = 8, PAGE = 16384;                   // ring pages, page bytes
-constexpr int MAXF = 2;                                 // pages in flight per loader wave (1: 3-9 % slower)
-constexpr uint32_t OOB = 0x80000000u;                   // buffer offset past every resource
+constexpr int TP = 64;   // token slots of a sample
+constexpr int RING = 8;  // ring pages
 
 // Shape of one configuration: G XCDs per group, NB samples per group.
 template <int G_, int NB_>
 struct Cfg {
-  static constexpr int G = G_, NB = NB_;
+  static constexpr int G = G_, NB = NB_, RING = pg::RING;
   static constexpr int NGRP = NX / G;
   static constexpr int HX = 8 / G;             // heads per XCD
   static constexpr int C = 4 / G;              // K windows of the O and down projections per XCD
@@ -83,11 +81,6 @@ struct Cfg {
   static_assert(LDS <= 160 * 1024, "LDS of one CU");
   static_assert(NB * HX * NKC == NR && NKC >= 2 && NB <= 2, "one attention item per rank");
 };
-constexpr uint32_t OFF_CTRL = 0, OFF_XFLAG = 1024;
-constexpr uint32_t OFF_DONE = 24;  // u32: groups of this launch that have finished
-static_assert(OFF_XFLAG + NX * NR * NCW * 8 <= kWsCounters, "flags stay below the fixup counters");
-static_assert(kWsGroupFlags + NX * NR * NCW * 8 <= kWsDataBase, "group flags stay below the data");
-
 __host__ __device__ constexpr uint32_t frag_off(int KS, int t, int k) {  // as in pi05_bs1.hip
   return (uint32_t)(((((t >> 4) * KS + (k >> 5)) * 16 + (t & 15)) * 4 + ((k >> 3) & 3)) * 16 + (k & 7) * 2);
 }
@@ -113,148 +106,13 @@ struct Params {
   int NL, Lp, Lmax, S, Tv, B, xt_rows;
 };
 
-extern __shared__ __attribute__((aligned(16))) unsigned char fg_lds[];
-
-struct Ctx {
-  int x, j, grp, r, wave, lane, lr, lq;
-  int ns;                 // samples of this group
+struct PCtx : Ctx {
   int an, ah, kbeg, kend, sbeg, nsfx, nun;  // attention item: slot, head, prefix keys, this step's keys, 64-key units
-  rsrc_t ws, rc, rs;
-  uint32_t xb, part;      // byte offsets of this XCD's block and this group's partial sums
-  uint32_t lds_addr;
-  unsigned* err;
-  uint64_t e, eg;         // epochs of this wave's latest XCD / group signal
+  rsrc_t rc, rs;
 };
 
-// Recompute lane-derived addresses per stage instead of keeping them live across the layer.
-__device__ __forceinline__ void launder(Ctx& c) { asm volatile("" : "+v"(c.lane), "+v"(c.lr), "+v"(c.lq)); }
-
-template <class K>
-__device__ __forceinline__ unsigned ctl_ld(int i) {
-  return __hip_atomic_load(reinterpret_cast<unsigned*>(fg_lds + K::L_CTL) + i, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-template <class K>
-__device__ __forceinline__ void ctl_st(int i, unsigned v) {
-  __hip_atomic_store(reinterpret_cast<unsigned*>(fg_lds + K::L_CTL) + i, v, __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ bool aborted(const Ctx& c) {
-  return __hip_atomic_load(c.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kErrSpin;
-}
-
-// ---------------------------------------------------------------- synchronisation
-// Signal: the wave drains its stores and publishes its epoch to its own flag (plain store, read by its
-// XCD). Waits are capped and set the sticky error bit, which makes every later wait return at once.
-__device__ __forceinline__ void xcd_signal(const Params& p, Ctx& c) {
-  __builtin_amdgcn_s_waitcnt(0);
-  c.e += 1;
-  if (c.lane == 0)
-    __hip_atomic_store(reinterpret_cast<uint64_t*>(p.ws + OFF_XFLAG) + (c.x * NR + c.r) * NCW + c.wave, c.e,
-                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-// Waits until ready(lane) holds in every lane of the wave; `load` returns whether the lane's flags are.
-template <class F>
-__device__ __forceinline__ void poll(const Ctx& c, const F& ok) {
-  if (aborted(c)) return;
-  for (unsigned it = 0;; ++it) {
-    if (__builtin_amdgcn_ballot_w64(!ok()) == 0) break;
-    if (it > kSpinCap) {
-      if (c.lane == 0) atomicOr(c.err, kErrSpin);
-      break;
-    }
-    __builtin_amdgcn_s_sleep(1);
-  }
-  asm volatile("" ::: "memory");  // loads after the wait stay after it
-}
-__device__ __forceinline__ bool flag_ge(u32x2 v, uint64_t e) { return (((uint64_t)v[1] << 32) | v[0]) >= e; }
-
-__device__ __forceinline__ void xcd_sync(const Params& p, Ctx& c) {
-  xcd_signal(p, c);
-  const uint32_t off = OFF_XFLAG + c.x * (NR * NCW * 8) + c.lane * 16;
-  poll(c, [&] {
-    const u32x4 v = ldb128<kCpSc1>(c.ws, off);
-    return flag_ge(u32x2{v[0], v[1]}, c.e) && flag_ge(u32x2{v[2], v[3]}, c.e);
-  });
-}
-// Waits until this wave index of the ranks in `mask` has passed the sync point this wave passed last.
-__device__ __forceinline__ void xcd_wait(const Ctx& c, uint32_t mask) {
-  const bool mine = c.lane < NR && ((mask >> (c.lane & 31)) & 1u);
-  const uint32_t off = mine ? OFF_XFLAG + ((c.x * NR + c.lane) * NCW + c.wave) * 8 : OOB;
-  poll(c, [&] { return !mine || flag_ge(ldb64<kCpSc1>(c.ws, off), c.e); });
-}
 // Token t of a sample is normed by rank t % 32, wave t / 16: the norm waves of this wave's tile.
 __device__ __forceinline__ void wait_norm_rows(const Ctx& c) { xcd_wait(c, c.wave & 1 ? 0xffff0000u : 0xffffu); }
-
-// Partial sums: published to the whole group. With G = 1 that is the XCD; otherwise the stores went out
-// with sc1 and so does the flag (its own array, read across XCDs).
-template <class K>
-__device__ __forceinline__ void part_signal(const Params& p, Ctx& c) {
-  if constexpr (K::G == 1) {
-    xcd_signal(p, c);
-  } else {
-    __builtin_amdgcn_s_waitcnt(0);
-    c.eg += 1;
-    if (c.lane == 0)
-      __hip_atomic_store(reinterpret_cast<uint64_t*>(p.ws + kWsGroupFlags) + (c.x * NR + c.r) * NCW + c.wave, c.eg,
-                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-}
-template <class K>
-__device__ __forceinline__ void part_wait(const Ctx& c) {
-  if constexpr (K::G == 1) {
-    xcd_wait(c, 0xffffffffu);
-  } else {
-    const uint32_t off = kWsGroupFlags + ((c.grp * K::G * NR + c.lane) * NCW + c.wave) * 8;
-    poll(c, [&] {
-      u32x2 v[K::G / 2];
-#pragma unroll
-      for (int i = 0; i < K::G / 2; i++) v[i] = ldb64<kCpSc1>(c.ws, off + i * 64 * NCW * 8);
-      bool ok = true;
-#pragma unroll
-      for (int i = 0; i < K::G / 2; i++) ok = ok && flag_ge(v[i], c.eg);
-      return ok;
-    });
-  }
-}
-// cache policy of partial-sum stores: they leave the XCD only with G > 1
-template <class K>
-constexpr int kCpPart = K::G == 1 ? kCpPlain : kCpSc1;
-
-// ---------------------------------------------------------------- weight ring
-template <class K>
-__device__ __forceinline__ void page_wait(const Ctx& c, int pg) {
-  for (unsigned it = 0;; ++it) {
-    const unsigned r0 = ctl_ld<K>(0), r1 = ctl_ld<K>(1);
-    if ((int)min(r0, r1) > pg || ctl_ld<K>(6)) break;
-    if (it > kSpinCap) {
-      ctl_st<K>(6, 1u);
-      if (c.lane == 0) atomicOr(c.err, kErrSpin);
-      break;
-    }
-    __builtin_amdgcn_s_sleep(1);
-  }
-  asm volatile("" ::: "memory");
-}
-template <class K>
-__device__ __forceinline__ void page_release(const Ctx& c, int upto) {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's LDS reads have returned
-  if (c.lane == 0) ctl_st<K>(2 + c.wave, (unsigned)upto);
-}
-
-// global_load_lds_dwordx4 with a wave-uniform base and a 32-bit lane offset: lane i copies 16 bytes to
-// LDS m0 + 16 i, so a fragment lands in MFMA lane order.
-__device__ __forceinline__ void dma16(const unsigned char* base, uint32_t voff, uint32_t lds) {
-  unsigned saved;
-  // (each half is cast to uint32_t before widening: readfirstlane returns int)
-  const uint64_t a = reinterpret_cast<uint64_t>(base);
-  const uint64_t u = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32)) << 32 |
-                     (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a);
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-               : "=&s"(saved)
-               : "v"(voff), "s"(u), "s"(__builtin_amdgcn_readfirstlane(lds))
-               : "memory");
-}
 
 // First row of QKV row tile rt of rank r (virtual rows: this XCD's heads, then k, then v).
 template <class K>
@@ -262,69 +120,12 @@ __device__ __forceinline__ int qkv_row(int j, int vr) {
   return vr < 256 * K::HX ? 256 * K::HX * j + vr : QD + (vr - 256 * K::HX);
 }
 
-#define FA_PG_VMCNT(n) (((n) & 15) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
-
-// Loader wave lw copies fragments 8 lw .. 8 lw + 7 of every page. Pages go out in the order the compute
-// waves read them: QKV, the chunk's K and V^T blocks, O, gate/up (PG passes), down; fragment F of a GEMM
-// stage with R row tiles is (k-step F / R, row tile F % R). A page needs its ring slot released by the
-// four compute waves and at most MAXF of this wave's pages in flight.
+// The pages of a layer: QKV, the chunk's segments of K and V^T, O, gate/up (PG passes), down.
 template <class K>
-struct Loader {
+struct Loader : LoaderBase<K> {
   const Params& p;
-  const Ctx& c;
-  int lw, pg = 0, done = 0;
-  bool ok = true;
-
-  __device__ __forceinline__ void complete_oldest() {
-    if (pg - done > 1)  // another page is in flight behind the oldest
-      __builtin_amdgcn_s_waitcnt(FA_PG_VMCNT(8));
-    else
-      __builtin_amdgcn_s_waitcnt(FA_PG_VMCNT(0));
-    static_assert(MAXF <= 2, "waits cover two pages in flight");
-    asm volatile("" ::: "memory");
-    ++done;
-    if (c.lane == 0) ctl_st<K>(lw, (unsigned)done);
-  }
-  __device__ __forceinline__ bool room() {
-    for (unsigned idle = 0;;) {
-      if (pg - done < MAXF) {
-        if (pg < RING) return true;
-        const unsigned m = min(min(ctl_ld<K>(2), ctl_ld<K>(3)), min(ctl_ld<K>(4), ctl_ld<K>(5)));
-        if ((int)m >= pg - RING + 1) return true;
-      }
-      if (done < pg) {
-        complete_oldest();
-        idle = 0;
-        continue;
-      }
-      if (ctl_ld<K>(6) || ++idle > kSpinCap) {
-        if (!ctl_ld<K>(6)) {
-          ctl_st<K>(6, 1u);
-          if (c.lane == 0) atomicOr(c.err, kErrSpin);
-        }
-        ok = false;
-        return false;
-      }
-      __builtin_amdgcn_s_sleep(1);
-    }
-  }
-  __device__ __forceinline__ uint32_t dst() const { return c.lds_addr + (uint32_t)(pg % RING) * PAGE + lw * 8192; }
-
-  // R row tiles of one GEMM stage: base(rt) = the tile's first row at the stage's first k
-  template <int R, int NP, class Base>
-  __device__ __forceinline__ void stage(uint32_t voff, const Base& base) {
-#pragma unroll 1
-    for (int i = 0; i < NP && ok; i++) {
-      if (!room()) return;
-      const uint32_t d = dst();
-#pragma unroll
-      for (int f = 0; f < 8; f++) {
-        const int F = 16 * i + 8 * lw + f, ks = F / R, rt = F - ks * R;
-        dma16(base(rt) + ks * 64, voff, d + f * 1024);
-      }
-      pg++;
-    }
-  }
+  const PCtx& c;
+  __device__ Loader(const Params& p_, const PCtx& c_, int lw_) : LoaderBase<K>(c_, lw_), p(p_), c(c_) {}
 
   __device__ void run() {
     const int NL = p.NL;
@@ -334,116 +135,56 @@ struct Loader {
     const uint32_t vstep = 16u * p.Lmax * 2;
     auto u8 = [](const bf16* q) { return reinterpret_cast<const unsigned char*>(q); };
 #pragma unroll 1
-    for (int li = 0; li < p.S * NL && ok; li++) {
+    for (int li = 0; li < p.S * NL && this->ok; li++) {
       const int l = li % NL;
       const unsigned char* w1 = u8(p.w1) + (size_t)l * 2560 * D * 2;
-      stage<K::RQ, K::PQ>(vq, [&](int rt) { return w1 + (size_t)qkv_row<K>(c.j, 16 * (K::RQ * c.r + rt)) * D * 2; });
+      this->template stage<K::RQ, K::RQ * K::KX>(vq, [&](int rt) { return w1 + (size_t)qkv_row<K>(c.j, 16 * (K::RQ * c.r + rt)) * D * 2; });
       const unsigned char* kb = u8(p.kcache) + ((size_t)b * NL + l) * p.Lmax * HD * 2;
       const unsigned char* vb = u8(p.vtcache) + ((size_t)b * NL + l) * HD * p.Lmax * 2;
 #pragma unroll 1
-      for (int u0 = 0; u0 < c.nun && ok; u0 += K::SEGU) {  // a segment: its K pages, then its V^T pages
+      for (int u0 = 0; u0 < c.nun && this->ok; u0 += K::SEGU) {  // a segment: its K pages, then its V^T pages
         const int np = 2 * min(K::SEGU, c.nun - u0);
 #pragma unroll 1
-        for (int i = 0; i < np; i++) {  // K: key tile lw, k-step f; keys past the chunk copy key 0 (masked later)
-          if (!room()) break;
-          int key = c.kbeg + 64 * u0 + 32 * i + 8 * (c.lr >> 2) + 4 * lw + (c.lr & 3);
+        for (int i = 0; i < np; i++) {  // K: key tile this->lw, k-step f; keys past the chunk copy key 0 (masked later)
+          if (!this->room()) break;
+          int key = c.kbeg + 64 * u0 + 32 * i + 8 * (c.lr >> 2) + 4 * this->lw + (c.lr & 3);
           if (key >= c.kend) key = 0;
-          const uint32_t d = dst();
+          const uint32_t d = this->dst();
 #pragma unroll
           for (int f = 0; f < 8; f++) dma16(kb + f * 64, (uint32_t)key * (HD * 2) + c.lq * 16, d + f * 1024);
-          pg++;
+          this->pg++;
         }
 #pragma unroll 1
-        for (int i = 0; i < np; i++) {  // V^T: dim tile 8 lw + f; an 8-key group that starts in the chunk
-          if (!room()) break;         // stays within the row (Lmax)
+        for (int i = 0; i < np; i++) {  // V^T: dim tile 8 this->lw + f; an 8-key group that starts in the chunk
+          if (!this->room()) break;         // stays within the row (Lmax)
           int kv = c.kbeg + 64 * u0 + 32 * i + 8 * c.lq;
           if (kv >= c.kend) kv = 0;
           const uint32_t vv = (uint32_t)c.lr * p.Lmax * 2 + kv * 2;
-          const uint32_t d = dst();
+          const uint32_t d = this->dst();
 #pragma unroll
-          for (int f = 0; f < 8; f++) dma16(vb + (size_t)(8 * lw + f) * vstep, vv, d + f * 1024);
-          pg++;
+          for (int f = 0; f < 8; f++) dma16(vb + (size_t)(8 * this->lw + f) * vstep, vv, d + f * 1024);
+          this->pg++;
         }
       }
       const unsigned char* wo = u8(p.wo) + ((size_t)l * D * QD + (size_t)16 * K::RP * rg * QD + 512 * (K::C * c.j + win)) * 2;
-      stage<K::RP, K::PO>(vo, [&](int rt) { return wo + (size_t)rt * 16 * QD * 2; });
+      this->template stage<K::RP, K::RP * K::KO>(vo, [&](int rt) { return wo + (size_t)rt * 16 * QD * 2; });
 #pragma unroll 1
       for (int q = 0; q < K::PG; q++) {
         const unsigned char* w2 =
             u8(p.w2) + ((size_t)l * 2 * FF + (size_t)c.j * (2 * FF / K::G) + 16 * (K::RG * c.r + K::RGP * q)) * D * 2;
-        stage<K::RGP, K::PGU / K::PG>(vq, [&](int rt) { return w2 + (size_t)rt * 16 * D * 2; });
+        this->template stage<K::RGP, K::RGP * K::KX>(vq, [&](int rt) { return w2 + (size_t)rt * 16 * D * 2; });
       }
       const unsigned char* w3 = u8(p.w3) + ((size_t)l * D * FF + (size_t)16 * K::RP * rg * FF + 1024 * (K::C * c.j + win)) * 2;
-      stage<K::RP, K::PD>(vd, [&](int rt) { return w3 + (size_t)rt * 16 * FF * 2; });
+      this->template stage<K::RP, K::RP * K::KD>(vd, [&](int rt) { return w3 + (size_t)rt * 16 * FF * 2; });
     }
-    if (ok)
-      while (done < pg) complete_oldest();
-    __builtin_amdgcn_s_waitcnt(0);
+    this->drain();
   }
 };
-
-// ---------------------------------------------------------------- GEMM (NB token tiles per wave)
-// acc[n][rt] = W[row tile rt][k] X[token][k] over KS k-steps, weights from ring pages pg0.. (fragment
-// F = ks R + rt), tokens from the workspace at xoff[n] + 1 KB per k-step (OOB: zeros). The operand
-// loads run two chunks of KC k-steps ahead (one chunk's MFMAs take 0.3-0.4 us, less than a loaded L2
-// round trip); A fragments are read from LDS in batches ahead of their MFMAs, each feeding NB of them;
-// pages are released as their last fragment is read.
-template <class K, int R, int KS>
-__device__ __forceinline__ void gemm(f32x4 (&acc)[K::NB][R], const Ctx& c, int pg0, const uint32_t (&xoff)[K::NB]) {
-  constexpr int NB = K::NB, KC = 8 / NB, NCK = KS / KC, NA = KC * R;
-  constexpr int AB = NA % 8 == 0 ? 8 : (NA % 5 == 0 ? 5 : 6);
-  static_assert(NA % AB == 0, "whole batches");
-  constexpr int CH = R * NB >= 4 ? 1 : 2;  // accumulator chains per row tile
-  f32x4 ac[CH][NB][R];
-#pragma unroll
-  for (int h = 0; h < CH; h++)
-#pragma unroll
-    for (int n = 0; n < NB; n++)
-#pragma unroll
-      for (int rt = 0; rt < R; rt++) ac[h][n][rt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  u32x4 xf[3][NB][KC];
-  auto load = [&](int ck) __attribute__((always_inline)) {
-#pragma unroll
-    for (int n = 0; n < NB; n++)
-#pragma unroll
-      for (int k = 0; k < KC; k++) xf[ck % 3][n][k] = ldb128<kCpSc1>(c.ws, xoff[n] + (ck * KC + k) * 1024);
-  };
-  load(0);
-  if (NCK > 1) load(1);
-#pragma unroll
-  for (int ck = 0; ck < NCK; ck++) {
-    if (ck + 2 < NCK) load(ck + 2);
-    page_wait<K>(c, pg0 + ((ck + 1) * NA - 1) / 16);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int h = 0; h < NA; h += AB) {
-      u32x4 af[AB];
-#pragma unroll
-      for (int q = 0; q < AB; q++) {
-        const int F = ck * NA + h + q;
-        af[q] = *reinterpret_cast<const u32x4*>(fg_lds + ((pg0 + F / 16) % RING) * PAGE + c.lane * 16 + (F % 16) * 1024);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int q = 0; q < AB; q++) {
-        const int k = (h + q) / R, rt = (h + q) % R;
-#pragma unroll
-        for (int n = 0; n < NB; n++) ac[k % CH][n][rt] = mfma16(af[q], xf[ck % 3][n][k], ac[k % CH][n][rt]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if ((ck + 1) * NA / 16 > ck * NA / 16) page_release<K>(c, pg0 + (ck + 1) * NA / 16);
-  }
-#pragma unroll
-  for (int n = 0; n < NB; n++)
-#pragma unroll
-    for (int rt = 0; rt < R; rt++) acc[n][rt] = CH == 2 ? ac[0][n][rt] + ac[CH - 1][n][rt] : ac[0][n][rt];
-}
 
 // Workspace offsets of the wave's token rows (tile (n, w)) of a fragment-ordered operand with KT k-steps,
 // from k-step ks0; rows past Tv or of an absent sample read zeros.
 template <class K>
-__device__ __forceinline__ void tok_off(const Params& p, const Ctx& c, uint32_t base, int KT, int ks0, uint32_t (&o)[K::NB]) {
+__device__ __forceinline__ void tok_off(const Params& p, const PCtx& c, uint32_t base, int KT, int ks0, uint32_t (&o)[K::NB]) {
   const int t = 16 * c.wave + c.lr;
 #pragma unroll
   for (int n = 0; n < K::NB; n++)
@@ -455,7 +196,7 @@ __device__ __forceinline__ void tok_off(const Params& p, const Ctx& c, uint32_t 
 // action projection and the Euler update. The wave norms token t = r + 32 (wave / 2) of every sample
 // (LDS slot 2 n + wave / 2); lane holds columns 4 lane + 256 k + i.
 template <class K, int MODE>
-__device__ __forceinline__ void stage_norm(const Params& p, const Ctx& c, uint32_t part, const float* gate,
+__device__ __forceinline__ void stage_norm(const Params& p, const PCtx& c, uint32_t part, const float* gate,
                                            const float* scale, const float* shift, float dt) {
   const int t = c.r + 32 * (c.wave >> 1);
   // the modulations do not depend on the wait; the partials of every sample are requested together
@@ -562,7 +303,7 @@ __device__ __forceinline__ void stage_norm(const Params& p, const Ctx& c, uint32
 
 // ---------------------------------------------------------------- QKV
 template <class K>
-__device__ __forceinline__ void stage_qkv(const Params& p, const Ctx& c, int li, int l, int pg0, bool last) {
+__device__ __forceinline__ void stage_qkv(const Params& p, const PCtx& c, int li, int l, int pg0, bool last) {
   constexpr int R = K::RQ;
   const int t = 16 * c.wave + c.lr;
   if (16 * c.wave >= p.Tv) {
@@ -574,7 +315,7 @@ __device__ __forceinline__ void stage_qkv(const Params& p, const Ctx& c, int li,
   f32x4 acc[K::NB][R];
   uint32_t xo[K::NB];
   tok_off<K>(p, c, K::X_XN, 32, 0, xo);
-  gemm<K, R, K::KX>(acc, c, pg0, xo);
+  gemm<K, R, K::KX, K::NB>(acc, c, pg0, xo);
 #pragma unroll
   for (int rt = 0; rt < R; rt++) {
     const int vr0 = 16 * (R * c.r + rt);  // wave-uniform: the tile lies within q, k or v
@@ -634,7 +375,7 @@ __device__ __forceinline__ void stage_qkv(const Params& p, const Ctx& c, int li,
 // K rows are permuted inside each 32-key block: row 4a + i of tile kt is key 8a + 4kt + i, so a lane's S^T
 // values of tiles (0, 1) are keys 8 lq .. 8 lq + 7, the P^T operand, and V^T fragments are read whole.
 template <class K>
-__device__ __forceinline__ void stage_att(const Params& p, const Ctx& c, int li, int pgk) {
+__device__ __forceinline__ void stage_att(const Params& p, const PCtx& c, int li, int pgk) {
   constexpr int NT = 4 * K::SEGU;  // key tiles of a segment
   if (16 * c.wave >= p.Tv || c.an >= c.ns) {
     page_release<K>(c, pgk + 4 * c.nun);
@@ -819,7 +560,7 @@ __device__ __forceinline__ void stage_att(const Params& p, const Ctx& c, int li,
 // Fragment id = (slot, head, k-step) of token tile w: wave w of rank r takes ids FPR r .. + FPR - 1 (with
 // G = 4: id r of ranks < 16). A lane owns one 16-byte slot (token 16 w + lane / 4, 8 dims).
 template <class K>
-__device__ __forceinline__ void stage_comb(const Params& p, const Ctx& c) {
+__device__ __forceinline__ void stage_comb(const Params& p, const PCtx& c) {
   constexpr int NF = K::FPR > 0 ? K::FPR : 1;
   const int id0 = c.r * NF;
   if (16 * c.wave >= p.Tv || id0 >= K::NB * K::HX * 8) return;
@@ -872,7 +613,7 @@ __device__ __forceinline__ void stage_comb(const Params& p, const Ctx& c) {
 
 // Stores the fp32 partial sums of the rank's rows (row group rg, window index wd of the group).
 template <class K>
-__device__ __forceinline__ void store_part(const Params& p, const Ctx& c, uint32_t part, int wd, int rg,
+__device__ __forceinline__ void store_part(const Params& p, const PCtx& c, uint32_t part, int wd, int rg,
                                            const f32x4 (&acc)[K::NB][K::RP]) {
   const int t = 16 * c.wave + c.lr;
   if (t >= p.Tv) return;
@@ -899,7 +640,7 @@ __device__ __forceinline__ uint32_t comb_ranks(int win) {
 }
 
 template <class K>
-__device__ __forceinline__ void stage_oproj(const Params& p, const Ctx& c, int pg0) {
+__device__ __forceinline__ void stage_oproj(const Params& p, const PCtx& c, int pg0) {
   if (16 * c.wave >= p.Tv) {
     page_release<K>(c, pg0 + K::PO);
     return;
@@ -909,12 +650,12 @@ __device__ __forceinline__ void stage_oproj(const Params& p, const Ctx& c, int p
   f32x4 acc[K::NB][K::RP];
   uint32_t xo[K::NB];
   tok_off<K>(p, c, K::X_ATTN, 8 * K::HX, 16 * win, xo);
-  gemm<K, K::RP, K::KO>(acc, c, pg0, xo);
+  gemm<K, K::RP, K::KO, K::NB>(acc, c, pg0, xo);
   store_part<K>(p, c, 0, K::C * c.j + win, rg, acc);
 }
 
 template <class K>
-__device__ __forceinline__ void stage_gu(const Params& p, const Ctx& c, int pg0) {
+__device__ __forceinline__ void stage_gu(const Params& p, const PCtx& c, int pg0) {
   if (16 * c.wave >= p.Tv) {
     page_release<K>(c, pg0 + K::PGU);
     return;
@@ -928,7 +669,7 @@ __device__ __forceinline__ void stage_gu(const Params& p, const Ctx& c, int pg0)
     // operand offsets are derived in each pass (hoisted out of the loop they spilled)
 #pragma unroll
     for (int n = 0; n < K::NB; n++) asm volatile("" : "+v"(xo[n]));
-    gemm<K, K::RGP, K::KX>(acc, c, pg0 + q * (K::PGU / K::PG), xo);
+    gemm<K, K::RGP, K::KX, K::NB>(acc, c, pg0 + q * (K::PGU / K::PG), xo);
     int t = 16 * c.wave + c.lr;
     asm volatile("" : "+v"(t));  // the store addresses are derived here, not kept live over the GEMM
     if (t >= p.Tv) continue;
@@ -954,7 +695,7 @@ __device__ __forceinline__ void stage_gu(const Params& p, const Ctx& c, int pg0)
 }
 
 template <class K>
-__device__ __forceinline__ void stage_dn(const Params& p, const Ctx& c, int pg0) {
+__device__ __forceinline__ void stage_dn(const Params& p, const PCtx& c, int pg0) {
   if (16 * c.wave >= p.Tv) {
     page_release<K>(c, pg0 + K::PD);
     return;
@@ -965,12 +706,12 @@ __device__ __forceinline__ void stage_dn(const Params& p, const Ctx& c, int pg0)
   f32x4 acc[K::NB][K::RP];
   uint32_t xo[K::NB];
   tok_off<K>(p, c, K::X_H, 128 / K::G, 32 * win, xo);
-  gemm<K, K::RP, K::KD>(acc, c, pg0, xo);
+  gemm<K, K::RP, K::KD, K::NB>(acc, c, pg0, xo);
   store_part<K>(p, c, K::PB - K::PB1, K::C * c.j + win, rg, acc);
 }
 
 // ---------------------------------------------------------------- instrumentation
-__device__ __forceinline__ void mark(const Params& p, const Ctx& c, int idx, uint64_t& t0) {
+__device__ __forceinline__ void mark(const Params& p, const PCtx& c, int idx, uint64_t& t0) {
   if (p.stage_cycles && blockIdx.x == 0 && c.wave == 0 && c.lane == 0) {
     const uint64_t now = __builtin_amdgcn_s_memrealtime();
     p.stage_cycles[idx] += now - t0;  // 0-7 stages N1 QKV ATT COMB O N2 GU DN, 8 final, 9 XCD barrier and signals
@@ -982,7 +723,7 @@ __device__ __forceinline__ void mark(const Params& p, const Ctx& c, int idx, uin
 template <int G, int NB>
 __global__ void __launch_bounds__(NTH, 1) pi05_group_kernel(Params p) {
   using K = Cfg<G, NB>;
-  Ctx c;
+  PCtx c;
   const int tid = threadIdx.x;
   c.x = blockIdx.x & 7;
   c.grp = c.x / G;
@@ -995,6 +736,7 @@ __global__ void __launch_bounds__(NTH, 1) pi05_group_kernel(Params p) {
   c.lq = c.lane >> 4;
   c.r = blockIdx.x >> 3;
   c.ws = make_rsrc(p.ws, K::WS);
+  c.wsp = p.ws;
   c.rc = make_rsrc(p.rope_cos, (uint32_t)(p.Tv * 128 * 4));
   c.rs = make_rsrc(p.rope_sin, (uint32_t)(p.Tv * 128 * 4));
   c.xb = K::OFF_XCD + (uint32_t)c.x * K::XB;
@@ -1016,7 +758,7 @@ __global__ void __launch_bounds__(NTH, 1) pi05_group_kernel(Params p) {
   const uint64_t seq = ld_flag(reinterpret_cast<const uint64_t*>(p.ws + OFF_CTRL));
   __syncthreads();  // the only workgroup barrier: LDS control words are initialised
   if (c.wave >= NCW) {
-    Loader<K> L{p, c, c.wave - NCW};
+    Loader<K> L(p, c, c.wave - NCW);
     L.run();
     return;
   }
@@ -1047,42 +789,42 @@ __global__ void __launch_bounds__(NTH, 1) pi05_group_kernel(Params p) {
           stage_norm<K, 1>(p, c, K::PB - K::PB1, mod_post - 6 * D + 2 * D, mod_in, mod_in + D, 0.f);
       }
       mark(p, c, 0, t0);
-      xcd_signal(p, c);
+      xcd_signal(c);
       launder(c);
       mark(p, c, 9, t0);
       stage_qkv<K>(p, c, li, l, pb, step == p.S - 1);
       mark(p, c, 1, t0);
-      xcd_sync(p, c);
+      xcd_sync(c);
       launder(c);
       mark(p, c, 9, t0);
       stage_att<K>(p, c, li, pb + K::PQ);
       mark(p, c, 2, t0);
-      xcd_signal(p, c);
+      xcd_signal(c);
       launder(c);
       mark(p, c, 9, t0);
       stage_comb<K>(p, c);
       mark(p, c, 3, t0);
-      xcd_signal(p, c);
+      xcd_signal(c);
       launder(c);
       mark(p, c, 9, t0);
       stage_oproj<K>(p, c, pb + K::PQ + 4 * c.nun);
       mark(p, c, 4, t0);
-      part_signal<K>(p, c);
+      part_signal<K>(c);
       launder(c);
       mark(p, c, 9, t0);
       if (nw) stage_norm<K, 1>(p, c, 0, mod_in + 2 * D, mod_post, mod_post + D, 0.f);
       mark(p, c, 5, t0);
-      xcd_signal(p, c);
+      xcd_signal(c);
       launder(c);
       mark(p, c, 9, t0);
       stage_gu<K>(p, c, pb + K::PQ + 4 * c.nun + K::PO);
       mark(p, c, 6, t0);
-      xcd_signal(p, c);
+      xcd_signal(c);
       launder(c);
       mark(p, c, 9, t0);
       stage_dn<K>(p, c, pb + K::PQ + 4 * c.nun + K::PO + K::PGU);
       mark(p, c, 7, t0);
-      part_signal<K>(p, c);
+      part_signal<K>(c);
     }
     if (nw) {
       const int li = step * NL + NL - 1;
@@ -1096,20 +838,7 @@ __global__ void __launch_bounds__(NTH, 1) pi05_group_kernel(Params p) {
     for (int n = 0; n < c.ns; n++)
       p.x_t[((size_t)(c.grp + n * K::NGRP) * p.xt_rows + t) * AD + c.lane] =
           reinterpret_cast<float*>(fg_lds + K::L_XT)[(2 * n + (c.wave >> 1)) * AD + c.lane];
-  // The launch sequence advances when the last group is done: the groups do not wait for one another, and
-  // a workgroup that starts late must still read this launch's number. (This wave has seen every wave of
-  // its group past the prologue.)
-  if (c.j == 0 && c.r == 0 && c.wave == 0 && c.lane == 0) {
-    unsigned* done = reinterpret_cast<unsigned*>(p.ws + OFF_DONE);
-    const unsigned groups = (unsigned)min(p.B, K::NGRP);
-    if (__hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == groups - 1) {
-      __hip_atomic_store(done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(reinterpret_cast<unsigned*>(p.ws + kWsOwner), kOwnerPi05Group, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(reinterpret_cast<uint64_t*>(p.ws + OFF_CTRL), seq + 1, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
+  if (c.j == 0 && c.r == 0 && c.wave == 0 && c.lane == 0) finish_group(p.ws, seq, (unsigned)min(p.B, K::NGRP), kOwnerPi05Group);
 }
 
 struct Choice {

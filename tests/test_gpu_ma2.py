@@ -57,6 +57,36 @@ def test_ma2_long_context(gpu, Lk, Tv):
     _check(C.make_case(NL=2, Lk=Lk, Tv=Tv, S=2, seed=Lk), gpu)
 
 
+# Every group shape (batch 1-4, 5-8, 9-16, two or four token tiles per sample) with groups of one sample, of
+# none and full, token counts on either side of the tiles, context chunks that are empty, ragged and
+# longer than one softmax segment, and the stage engine past them (17). Four steps: at two, bf16 operands
+# alone leave 1.4e-3 mean-abs, and 1.1e-3 to 2.1e-3 over a sample of 30 values (the stage engine's 17 x 5
+# tokens); the error falls with the step length.
+@pytest.mark.parametrize("B,Lk,Tv,adim", [(1, 33, 33, 6), (2, 1, 32, 6), (3, 700, 16, 6), (4, 1100, 64, 6),
+                                          (5, 129, 17, 32), (8, 513, 49, 6), (9, 64, 30, 6), (16, 300, 31, 6),
+                                          (12, 65, 50, 1), (17, 50, 5, 6)])
+def test_ma2_group_shapes(gpu, B, Lk, Tv, adim):
+    _check(C.make_case(NL=2, Lk=Lk, Tv=Tv, S=4, adim=adim, batch=B, seed=B + Lk + Tv), gpu)
+
+
+def test_ma2_groups_repeat_on_one_workspace(gpu):
+    """Launches of different group shapes and of the stage engine (a workspace with no room for the groups)
+    on one workspace, each against its first result."""
+    import torch
+    cs = [C.make_case(NL=1, Lk=90, Tv=Tv, S=2, batch=B, seed=B) for B, Tv in ((2, 20), (3, 40), (6, 20), (6, 40), (12, 20))]
+    n = max(ma2.workspace(gpu, c["batch"], c["Tv"], 96).numel() for c in cs)
+    raw = torch.zeros(n + 256, dtype=torch.uint8, device=gpu)
+    ws = raw[(-raw.data_ptr()) % 256:][:n]
+    first = {}
+    for r in range(2):
+        for i, c in enumerate(cs):
+            out = C.run_gpu(c, gpu, ws=ws)
+            assert ma2.read_status(ws) == 0
+            assert np.array_equal(out, first.setdefault(i, out))
+    out = C.run_gpu(cs[0], gpu, ws=ws[:(8 << 20)])
+    assert np.abs(out - first[0]).max() <= MAX_ABS
+
+
 def test_ma2_batch16(gpu):
     """The MolmoAct2 benchmark workload at batch 16 (the large-tile path) at full depth, 36 layers x 10 steps, every
     sample against the oracle (benchmarks/molmoact2/eval_numerics.py:147-159 is the reference's
