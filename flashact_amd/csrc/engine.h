@@ -225,8 +225,8 @@ __device__ __forceinline__ u32x4 pack_pre(const E& e, int n, f32x4 v, const type
 // rows r, r+16, r+32, r+48 (k step = 256 B each, 16 lanes per row) and lands them as 4 x 256 B at
 // LDS pitch 1040 B. An MFMA fragment (16 rows of one 16-row block, 32 k) then reads row r from
 // copy r at 1040 r + 256 (block % 4) + 64 ks + 16 q: the 16 rows fall in 16 different bank groups.
-// Ring of RD steps (2, or 3 where three fit the kernel's LDS: two steps then stay in flight while one
-// computes), one workgroup barrier per step. Rows m >= M copy row 0 (results discarded).
+// Ring of RD steps (2, or 3 or 4 where they fit the kernel's LDS: RD - 1 steps then stay in flight while
+// one computes), one workgroup barrier per step. Rows m >= M copy row 0 (results discarded).
 // With AF the activations are in MFMA fragment order instead (fragment (token block tb, k-step kk) =
 // 1 KB at (tb lda / 32 + kk) * 1024, lane l = lr + 16 q holding token lr, k 8q..8q+7 at 16 l): copy f
 // of a step is fragment (token block f / 4, k-step f % 4), one contiguous 1 KB, and lands whole in slot
@@ -315,9 +315,12 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int m0, int n0, int
   }
   issue(0);
   if (RD > 2 && ns > 1) issue(1);
+  if (RD > 3 && ns > 2) issue(2);
 #pragma unroll 1
   for (int s = 0; s < ns; s++) {
-    if (RD > 2 && s + 1 < ns)
+    if (RD > 3 && s + 2 < ns)
+      vm_wait<2 * S::IPW>();  // the copies of steps s + 1 and s + 2 (the last issued) may still be in flight
+    else if (RD > 2 && s + 1 < ns)
       vm_wait<S::IPW>();  // step s + 1's copies (the last issued) may still be in flight
     else
       vm_wait<0>();
@@ -463,7 +466,7 @@ __device__ __forceinline__ void gemm_stage(const GemmArgs& g, int N, int K, int 
 }
 
 // ---------------------------------------------------------------- direct-operand GEMM tiles
-// gemm_tile_d<TW, WM>: a (16 WM TW)-token x 128-feature tile whose token operand skips LDS. The NWAVE
+// gemm_tile_d<TW, WM, BN>: a (16 WM TW)-token x BN-feature tile (BN = 128 or 64) whose token operand skips LDS. The NWAVE
 // waves form TW rows along the tokens and NWAVE / TW columns along the features; wave (wt, wf) computes
 // WM token blocks x WN feature blocks of 16 x 16. The tall tile (TW = NWAVE, WM = 4: 256 x 128 with 4
 // waves, 512 x 128 with 8; a wave holds 64 tokens x 128 features, 32 MFMAs per 32-k sub-step for 12
@@ -501,20 +504,21 @@ template <class E>
 struct IsStaged<E, std::void_t<decltype(E::kStaged)>> : std::bool_constant<E::kStaged && (E::kRowBytes > 0)> {};
 
 // LDS bytes of gemm_tile_d<TW, WM>'s staged epilogue (8 output bytes per 4 features, 16 B row padding)
-template <int TW, int WM>
+template <int TW, int WM, int BN = 128>
 constexpr uint32_t staged_d_lds() {
-  return (uint32_t)NWAVE * 16 * WM * (128 / (NWAVE / TW) / 4 * 8 + 16);
+  return (uint32_t)NWAVE * 16 * WM * (BN / (NWAVE / TW) / 4 * 8 + 16);
 }
 
 // Epilogue: epi(n, m, v) with features n..n+3 of token m (m < M only); an epilogue with a Pre type
 // (gemm_tile's interface) gets epi(n, m, v, pre) with every block's pre fetched before the first call.
-template <int TW, int WM, class Epi>
+template <int TW, int WM, int BN = 128, class Epi>
 __device__ __forceinline__ void gemm_tile_d(const GemmArgsF& g, int m0, int n0, int k0, int k1, Epi& epi) {
   static_assert(NWAVE % TW == 0 && (NWAVE / TW == 1 || NWAVE / TW == 2), "TW waves along the tokens");
   // FW waves along the features; CPW weight copies per wave and step, CPK of them in each of the
   // step's first two sub-steps (one every JM feature blocks)
-  constexpr int FW = NWAVE / TW, WN = 8 / FW, NA = 4 * WM, CPW = 32 / NWAVE, CPK = CPW / 2, JM = WN / CPK;
-  static_assert(JM >= 1 && WN % CPK == 0, "copy schedule");
+  constexpr int FW = NWAVE / TW, WN = BN / 16 / FW, NA = 4 * WM, CPW = BN / 4 / NWAVE, CPK = CPW / 2, JM = WN / CPK;
+  static_assert(BN == 64 || BN == 128, "whole 64-row weight groups");
+  static_assert(CPK >= 1 && CPW % 2 == 0 && JM >= 1 && WN % CPK == 0, "copy schedule");
   const int w = wave_id(), lane = lane_id(), lr = lane & 15, lq = lane >> 4;
   const int wt = w / FW, wf = w % FW;
   // copy f = w + NWAVE j of a step: rows 64 (f / 16) + 16 lq + f % 16 of the tile, 16 B per lane
@@ -524,7 +528,8 @@ __device__ __forceinline__ void gemm_tile_d(const GemmArgsF& g, int m0, int n0, 
   const uint32_t wlo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)wb);
   const uint32_t whi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(wb >> 32));
   const void* wbase = reinterpret_cast<const void*>(((uint64_t)whi << 32) | wlo);
-  const uint32_t wlane = (uint32_t)((16 * lq * g.ldw + k0 + 8 * lr) * 2);
+  uint32_t wlane = (uint32_t)((16 * lq * g.ldw + k0 + 8 * lr) * 2);
+  asm volatile("" : "+v"(wlane));  // one VGPR: the copies' lane offsets, precomputed, spilled a register
   const int tb0 = (m0 >> 4) + WM * wt;  // the wave's first token block
   const uint32_t abase = (uint32_t)(((size_t)tb0 * g.KF + (k0 >> 5)) * 1024 + lane * 16);
   const int ns = (k1 - k0) >> 7;
@@ -600,7 +605,7 @@ __device__ __forceinline__ void gemm_tile_d(const GemmArgsF& g, int m0, int n0, 
     // stores 16 contiguous bytes of a row, so an instruction writes whole row segments (four 256-byte
     // rows of bf16 partials) instead of 8 B into each of 16 rows. The kernel's LDS must hold
     // staged_d_lds<TW, WM>() bytes.
-    constexpr int OB = Epi::kRowBytes, RB = 128 / FW / 4 * OB, RP = RB + 16, WR = 16 * WM;
+    constexpr int OB = Epi::kRowBytes, RB = BN / FW / 4 * OB, RP = RB + 16, WR = 16 * WM;
     static_assert(OB == 8 && RB % 16 == 0 && 64 % (RB / 16) == 0, "8 output bytes per 4 features");
     __syncthreads();  // every wave's last MFMAs have read the ring
     if (16 * tb0 < g.M) {
@@ -620,7 +625,7 @@ __device__ __forceinline__ void gemm_tile_d(const GemmArgsF& g, int m0, int n0, 
       for (int r = lane / TPR; r < WR; r += RPP) {
         const int m = m0 + WR * wt + r;
         if (m < g.M)
-          st_b128(epi.ws, epi.row_off(m, n0 + 128 / FW * wf) + (uint32_t)(tc * 16), lds128(base + (uint32_t)(r * RP + tc * 16)));
+          st_b128(epi.ws, epi.row_off(m, n0 + BN / FW * wf) + (uint32_t)(tc * 16), lds128(base + (uint32_t)(r * RP + tc * 16)));
       }
     }
     __syncthreads();  // the staged rows are read before the next tile's copies land
@@ -654,18 +659,18 @@ __device__ __forceinline__ void gemm_tile_d(const GemmArgsF& g, int m0, int n0, 
   }
 }
 
-// Every (16 WM TW) x 128 tile of an [M x N] GEMM (N a multiple of 128), K split into `ksplit` ranges
+// Every (16 WM TW) x BN tile of an [M x N] GEMM (N a multiple of BN), K split into `ksplit` ranges
 // (multiples of 128); items m-tile fastest, as in gemm_stage. The epilogue gets the split in epi.split.
-template <int TW, int WM, class Epi>
+template <int TW, int WM, int BN = 128, class Epi>
 __device__ __forceinline__ void gemm_stage_d(const GemmArgsF& g, int N, int K, int ksplit, Epi& epi) {
   constexpr int BM = 16 * WM * TW;
-  const int nm = (g.M + BM - 1) / BM, nn = N / 128;
+  const int nm = (g.M + BM - 1) / BM, nn = N / BN;
   const int items = nm * nn * ksplit, kc = K / ksplit;
 #pragma unroll 1
   for (int it = vwg(); it < items; it += NWG) {
     const int mt = it % nm, rest = it / nm, nt = rest % nn, sp = rest / nn;
     epi.split = sp;
-    gemm_tile_d<TW, WM>(g, mt * BM, nt * 128, sp * kc, sp * kc + kc, epi);
+    gemm_tile_d<TW, WM, BN>(g, mt * BM, nt * BN, sp * kc, sp * kc + kc, epi);
   }
 }
 

@@ -15,10 +15,11 @@
 //   O    [M x 2048] = attn Wo^T, K split 2 ways -> bf16 partials
 // O, GU and DN read their token operand (attn, xn after N2, h) in MFMA fragment order.
 //   N2   x += sum(partials); xn = rms(x) (1 + w_post), written in MFMA fragment order
-//   GU   [M x 32768] = xn Wgu^T (gate/up rows interleaved, 512 x 128 tiles) -> h = gelu_tanh(g) u
+//   GU   [M x 32768] = xn Wgu^T (gate/up rows interleaved, tall tiles) -> h = gelu_tanh(g) u
 //        [M x 16384], fragment order
-//   DN   [M x 2048] = h Wdn^T (512 x 128 tiles), K split 8 ways -> bf16 partials
-// The last layer stops after QKV: its attention and MLP outputs reach no cache entry.
+//   DN   [M x 2048] = h Wdn^T (tall tiles), K split 8 ways -> bf16 partials
+// The last layer stops after QKV: its attention and MLP outputs reach no cache entry. Tile shapes follow
+// the token count (Plan).
 // Two waves per SIMD (8 per workgroup): the tall MLP tiles keep the MFMA pipe busy about 1.4x as long
 // as one wave per SIMD can, at a budget of 256 registers per lane in every stage.
 #define FA_ENG_NWAVE 8
@@ -37,6 +38,43 @@ constexpr int QKVN = QD + 2 * HD;  // 2560 projection rows
 constexpr int KS_O = 2, KS_DN = 8;  // K splits of the O and down projections
 constexpr int MAX_TOKENS = 16384;  // batch x Lp
 static_assert((size_t)NH * MAX_TOKENS < (1u << 20), "divmod_u: the combine rows stay below 2^20");
+
+// Tile shapes of the four GEMM stages: QKV and O tiles of 32 QM x 32 QN and 32 OM x 32 ON (tokens x
+// features, gemm_tile, rings of QR and OR steps), gate/up tiles of 128 GW x 128 and down tiles of
+// 128 DW x DB (gemm_tile_d). A stage's items (tiles x K splits) run in rounds of NWG, and a round costs
+// about the same however few of its workgroups have work (its time is the tile's own chain of k steps),
+// so fewer tokens want smaller tiles, and a count just past a multiple of a tile's height a shape that
+// leaves no nearly empty round. K splits and the k order are the same in every plan, and so are results.
+// One kernel per plan: a single kernel that switched shapes ran the plan of M = 968 2.3 % slower than the
+// kernel that holds only that one.
+template <int QM_, int QN_, int QR_, int OM_, int ON_, int OR_, int GW_, int DW_, int DB_>
+struct Plan {
+  static constexpr int QM = QM_, QN = QN_, QR = QR_, OM = OM_, ON = ON_, OR = OR_, GW = GW_, DW = DW_, DB = DB_;
+  // µs of one round of the stage, measured in this kernel (a second round costs no more than the first).
+  // Deeper rings pay on the smaller tiles (QKV 64 x 64, 2 -> 4 steps: 15.4 -> 11.6 µs; O: 7.6 -> 5.6).
+  static constexpr float q_us() { return QN == 2 ? (QM == 2 ? 11.5f : 15.7f) : (QM == 2 ? 18.5f : 24.0f); }
+  static constexpr float o_us() { return ON == 4 ? 11.8f : OM == 2 ? 5.6f : OM == 3 ? 6.6f : 8.0f; }
+  static constexpr float g_us() { return GW == 1 ? 21.0f : GW == 2 ? 26.5f : GW == 3 ? 37.0f : 47.5f; }
+  static constexpr float d_us() {
+    return DB == 64 ? (DW == 1 ? 16.5f : DW == 2 ? 20.0f : 26.0f) : DW == 2 ? 27.0f : DW == 3 ? 37.0f : 45.0f;
+  }
+  static float cost(int M) {  // µs of a layer's GEMM stages
+    auto rounds = [&](int bm, int tiles_n) { return (float)(((M + bm - 1) / bm * tiles_n + NWG - 1) / NWG); };
+    return rounds(32 * QM, QKVN / (32 * QN)) * q_us() + rounds(32 * OM, D / (32 * ON) * KS_O) * o_us() +
+           rounds(128 * GW, 2 * FF / 128) * g_us() + rounds(128 * DW, D / DB * KS_DN) * d_us();
+  }
+};
+// Prefill of one sample, PlanMax for every size -> the plan taken (ms): Lp 60 2.79 -> 1.87, 129 2.80 -> 2.01,
+// 293 3.04 -> 2.32, 400 3.17 -> 2.66, 561 3.80 -> 3.33, 968 the same plan, 1100 6.16 -> 5.66, 1300 6.92 -> 6.42;
+// four samples of 561: 9.98 -> 9.59. Weights alone take 0.74 ms at 5 TB/s: small counts are bound by the
+// chain of seven grid barriers and k-step chains per layer, large ones by the matrix cores.
+using Plan128 = Plan<2, 2, 4, 2, 2, 4, 1, 1, 64>;
+using Plan256 = Plan<2, 2, 4, 2, 2, 4, 2, 2, 64>;
+using Plan384 = Plan<2, 2, 4, 3, 2, 3, 3, 3, 64>;
+using Plan512 = Plan<3, 2, 3, 4, 2, 3, 4, 2, 128>;
+using Plan768 = Plan<2, 4, 3, 4, 4, 2, 3, 3, 128>;
+using Plan1152 = Plan<3, 4, 2, 4, 4, 2, 3, 3, 128>;
+using PlanMax = Plan<3, 4, 2, 4, 4, 2, 4, 4, 128>;
 
 struct Layout {
   int B, Tv, M, MP, NQT, NKC;
@@ -232,11 +270,14 @@ __device__ __forceinline__ void stage_norm(const Params& p, rsrc_t ws, rsrc_t xi
   }
 }
 
-constexpr uint32_t LDS_GEMM = GemmShape<4, 4>::LDS > TALL_LDS ? GemmShape<4, 4>::LDS : TALL_LDS;
-constexpr uint32_t LDS_ATTG = LDS_GEMM > ATT_LDS ? LDS_GEMM : ATT_LDS;
-constexpr uint32_t LDS_STAGE = staged_d_lds<NWAVE, 4>();  // the down projection's staged rows
-constexpr uint32_t LDS_BYTES = LDS_ATTG > LDS_STAGE ? LDS_ATTG : LDS_STAGE;
-static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
+constexpr uint32_t lds_max(uint32_t a, uint32_t b) { return a > b ? a : b; }
+template <class PL>
+constexpr uint32_t lds_bytes() {
+  const uint32_t gemm = lds_max(lds_max(PL::QR * GemmShape<PL::QM, PL::QN>::STEP, PL::OR * GemmShape<PL::OM, PL::ON, true>::STEP),
+                                lds_max(TALL_LDS, staged_d_lds<NWAVE, PL::DW, PL::DB>()));
+  static_assert(lds_max(gemm, ATT_LDS) <= 160 * 1024, "LDS budget");
+  return lds_max(gemm, ATT_LDS);
+}
 
 __device__ __forceinline__ void mark(const Params& p, int idx, uint64_t& t0) {
   if (p.stage_cycles) {  // t0 moves in every wave: a value set under the thread test would live in VGPRs
@@ -246,6 +287,7 @@ __device__ __forceinline__ void mark(const Params& p, int idx, uint64_t& t0) {
   }
 }
 
+template <class PL>
 __global__ void __launch_bounds__(NTHR, 1) prefill_kernel(Params p) {
   const Layout& L = p.L;
   const rsrc_t ws = rsrc_all(p.ws);
@@ -284,7 +326,7 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_kernel(Params p) {
     {
       EpiQKV e{ws, kc, vc, p.rope_cos, p.rope_sin, (uint32_t)L.qf, L.NQT, p.Tv, NL, p.Lmax, p.Lp, l, 0, rtv};
       gx.W = p.wqkv + (size_t)l * QKVN * D;
-      gemm_stage<3, 4>(gx, QKVN, D, 1, e);  // 96-token tiles: 220 items (160 of 128): QKV 29.1 -> 26.3 us per layer
+      gemm_stage<PL::QM, PL::QN, false, PL::QR>(gx, QKVN, D, 1, e);
     }
     mark(p, 1, t0);
     if (l == NL - 1) break;  // the last layer's K/V are in the caches
@@ -301,7 +343,7 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_kernel(Params p) {
     {
       EpiPart e{{}, ws, (uint32_t)L.part, L.MP, 0};
       ga.W = p.wo + (size_t)l * D * QD;
-      gemm_stage<4, 4, true>(ga, D, QD, KS_O, e);
+      gemm_stage<PL::OM, PL::ON, true, PL::OR>(ga, D, QD, KS_O, e);
     }
     mark(p, 4, t0);
     grid_sync(grid);
@@ -313,7 +355,7 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_kernel(Params p) {
     {
       EpiGeluF e{ws, (uint32_t)L.h, 0};
       gxf.W = p.wgu + (size_t)l * 2 * FF * D;
-      gemm_stage_tall(gxf, 2 * FF, D, 1, e);
+      gemm_stage_d<NWAVE, PL::GW>(gxf, 2 * FF, D, 1, e);
     }
     mark(p, 6, t0);
     grid_sync(grid);
@@ -321,7 +363,7 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_kernel(Params p) {
     {
       EpiPartB e{ws, (uint32_t)L.part, L.MP, 0};
       ghf.W = p.wdn + (size_t)l * D * FF;
-      gemm_stage_tall(ghf, D, FF, KS_DN, e);
+      gemm_stage_d<NWAVE, PL::DW, PL::DB>(ghf, D, FF, KS_DN, e);
     }
     mark(p, 7, t0);
     grid_sync(grid);
@@ -330,6 +372,24 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_kernel(Params p) {
   if (grid_thread0())
     __hip_atomic_store(reinterpret_cast<uint64_t*>(p.ws + OFF_CTRL), seq + 1, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
+}
+
+struct Launch {
+  const void* fn;
+  uint32_t lds;
+};
+// The plan of the lowest cost at M tokens; of equal ones the larger tiles, which read fewer operand bytes.
+template <class First, class... Rest>
+inline Launch pick_plan(int M, float best, Launch k) {
+  const float c = First::cost(M);
+  if (c < best) best = c, k = Launch{(const void*)prefill_kernel<First>, lds_bytes<First>()};
+  if constexpr (sizeof...(Rest) > 0)
+    return pick_plan<Rest...>(M, best, k);
+  else
+    return k;
+}
+inline Launch pick(int M) {
+  return pick_plan<PlanMax, Plan1152, Plan768, Plan512, Plan384, Plan256, Plan128>(M, 1e30f, Launch{});
 }
 
 }  // namespace pf
@@ -380,7 +440,8 @@ extern "C" int fa_pi05_prefill(const fa_prefill_args* a, fa_stream_t stream) {
   if (need == 0 || a->workspace_bytes < need)
     return host::fail(FA_ERR_INVALID_ARG, "fa_pi05_prefill: workspace_bytes=%zu < required %zu", a->workspace_bytes,
                       need);
-  int rc = host::check_device((const void*)prefill_kernel, NTHR, LDS_BYTES, NWG, "fa_pi05_prefill");
+  const Launch k = pick(a->batch * a->Lp);
+  int rc = host::check_device(k.fn, NTHR, k.lds, NWG, "fa_pi05_prefill");
   if (rc != FA_OK) return rc;
   Params p;
   p.wqkv = static_cast<const bf16*>(a->wqkv);
@@ -403,5 +464,5 @@ extern "C" int fa_pi05_prefill(const fa_prefill_args* a, fa_stream_t stream) {
   p.Tv = a->Lp;
   p.B = a->batch;
   void* args[] = {&p};
-  return host::coop_launch((const void*)prefill_kernel, NWG, NTHR, args, LDS_BYTES, stream, "fa_pi05_prefill");
+  return host::coop_launch(k.fn, NWG, NTHR, args, k.lds, stream, "fa_pi05_prefill");
 }

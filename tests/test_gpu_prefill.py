@@ -119,6 +119,18 @@ def test_prefill_batch_matches_single(gpu):
         assert torch.equal(k1[0], kb[b]) and torch.equal(v1[0], vb[b])
 
 
+def test_prefill_tile_plans(gpu):
+    """Every tile plan and both sides of each of its edges, tokens without neighbours (Lp = 1, so M = batch):
+    the K splits and the k order do not depend on the plan, so a token's K and V are the same bits in all."""
+    M = 1153
+    c = C.make_case(NL=2, Lp=1, batch=M, seed=12)
+    g = C.gpu_weights(c, gpu)
+    kr, vr = C.run_gpu(c, gpu, g)
+    for n in (2, 64, 65, 128, 129, 256, 257, 384, 385, 512, 513, 768, 769, 1024, 1025, 1152):
+        k, v = C.run_gpu(c, gpu, g, samples=list(range(M - n, M)))
+        assert torch.equal(k, kr[M - n:]) and torch.equal(v, vr[M - n:]), n
+
+
 def test_prefill_deterministic(gpu):
     c = C.make_case(NL=2, Lp=333, seed=4)
     g = C.gpu_weights(c, gpu)
