@@ -159,7 +159,7 @@ __device__ __forceinline__ void page_release(const Ctx& c, int upto) {
 }
 
 // global_load_lds_dwordx4 with a wave-uniform base and a 32-bit lane offset: lane i copies 16 bytes to
-// LDS m0 + 16 i, so a fragment lands in MFMA lane order.
+// LDS m0 + 16 i (fragments in the order of copy_row / copy_chunk).
 __device__ __forceinline__ void dma16(const unsigned char* base, uint32_t voff, uint32_t lds) {
   unsigned saved;
   // (each half is cast to uint32_t before widening: readfirstlane returns int)
@@ -261,6 +261,7 @@ __device__ __forceinline__ void gemm(f32x4 (&acc)[NB][R], const Ctx& c, int pg0,
     for (int n = 0; n < NB; n++)
 #pragma unroll
       for (int rt = 0; rt < R; rt++) ac[h][n][rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint32_t fo = frag_slot(c.lr, c.lq);
   u32x4 xf[3][NB][KC];
   auto load = [&](int ck) __attribute__((always_inline)) {
 #pragma unroll
@@ -281,7 +282,7 @@ __device__ __forceinline__ void gemm(f32x4 (&acc)[NB][R], const Ctx& c, int pg0,
 #pragma unroll
       for (int q = 0; q < AB; q++) {
         const int F = ck * NA + h + q;
-        af[q] = *reinterpret_cast<const u32x4*>(fg_lds + ((pg0 + F / 16) % K::RING) * PAGE + c.lane * 16 + (F % 16) * 1024);
+        af[q] = *reinterpret_cast<const u32x4*>(fg_lds + ((pg0 + F / 16) % K::RING) * PAGE + fo + (F % 16) * 1024);
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll

@@ -101,7 +101,7 @@ struct MCtx : Ctx {
 
 // Byte offset of (token t of its tile, column k) inside a tile of a fragment-ordered operand.
 __device__ __forceinline__ uint32_t tfrag(int t, int k) {
-  return (uint32_t)((((k >> 5) * 16 + (t & 15)) * 4 + ((k >> 3) & 3)) * 16 + (k & 7) * 2);
+  return (uint32_t)((((k >> 5) * 4 + ((k >> 3) & 3)) * 16 + (t & 15)) * 16 + (k & 7) * 2);
 }
 // The wave's i-th token tile: sample slot, tile of the sample, index among all.
 template <class K>
@@ -129,7 +129,8 @@ struct Loader : LoaderBase<K> {
   __device__ void run() {
     const int NL = p.NL;
     auto u8 = [](const bf16* q) { return reinterpret_cast<const unsigned char*>(q); };
-    const uint32_t vx = c.lr * (D * 2) + c.lq * 16, vd = c.lr * (FF * 2) + c.lq * 16;
+    const int cr = copy_row(c.lane), cq = copy_chunk(c.lane);
+    const uint32_t vx = cr * (D * 2) + cq * 16, vd = cr * (FF * 2) + cq * 16;
     const int win = c.r / K::NRG, rg = c.r % K::NRG;
     const bool po = c.r < K::NRG * K::C;
     const int b = c.grp + c.an * K::NGRP, hg = K::HX * c.j + c.ah;
@@ -162,14 +163,14 @@ struct Loader : LoaderBase<K> {
 #pragma unroll
           for (int f = 0; f < 8; f++) {
             const int ff = f % 6, kt = ff / 3, ks = ff - 3 * kt;
-            int key = k0 + 8 * (c.lr >> 2) + 4 * kt + (c.lr & 3);
+            int key = k0 + 8 * (cr >> 2) + 4 * kt + (cr & 3);
             if (key >= c.kend) key = 0;
-            dma16(kb + ks * 64, (uint32_t)key * (D * 2) + c.lq * 16, d + f * 1024);
+            dma16(kb + ks * 64, (uint32_t)key * (D * 2) + cq * 16, d + f * 1024);
           }
         } else {
-          int kg = k0 + 8 * c.lq;
+          int kg = k0 + 8 * cq;
           if (kg >= c.kend) kg = 0;
-          const uint32_t vv = (uint32_t)c.lr * p.Lkmax * 2 + kg * 2;
+          const uint32_t vv = (uint32_t)cr * p.Lkmax * 2 + kg * 2;
 #pragma unroll
           for (int f = 0; f < 8; f++) dma16(vb + (size_t)(f % 6) * 16 * p.Lkmax * 2, vv, d + f * 1024);
         }
@@ -199,7 +200,7 @@ __device__ __forceinline__ void tok_off(const Params& p, const Ctx& c, uint32_t 
 #pragma unroll
   for (int i = 0; i < K::NI; i++)
     o[i] = t < p.Tv && slot_of<K>(c, i) < c.ns
-               ? c.xb + base + (uint32_t)((tidx<K>(c, i) * KT + ks0) * 1024 + (c.lr * 4 + c.lq) * 16)
+               ? c.xb + base + (uint32_t)((tidx<K>(c, i) * KT + ks0) * 1024 + c.lane * 16)
                : OOB;
 }
 
@@ -558,7 +559,7 @@ __device__ __forceinline__ void stage_catt(const Params& p, const MCtx& c, int p
       page_wait<K>(c, pgk + bi);
       u32x4 kf[6];
 #pragma unroll
-      for (int f = 0; f < 6; f++) kf[f] = *reinterpret_cast<const u32x4*>(fg_lds + ((pgk + bi) % K::RING) * PAGE + f * 1024 + c.lane * 16);
+      for (int f = 0; f < 6; f++) kf[f] = *reinterpret_cast<const u32x4*>(fg_lds + ((pgk + bi) % K::RING) * PAGE + f * 1024 + frag_slot(c.lr, c.lq));
 #pragma unroll
       for (int kt = 0; kt < 2; kt++) {
         f32x4 a = {0.f, 0.f, 0.f, 0.f};
@@ -602,7 +603,7 @@ __device__ __forceinline__ void stage_catt(const Params& p, const MCtx& c, int p
       u32x4 vf[6];
 #pragma unroll
       for (int f = 0; f < 6; f++)
-        vf[f] = *reinterpret_cast<const u32x4*>(fg_lds + ((pgk + bi) % K::RING) * PAGE + 8192 + f * 1024 + c.lane * 16);
+        vf[f] = *reinterpret_cast<const u32x4*>(fg_lds + ((pgk + bi) % K::RING) * PAGE + 8192 + f * 1024 + frag_slot(c.lr, c.lq));
       if (nv < 32) {
         const int q = min(max(nv - 8 * c.lq, 0), 8);
 #pragma unroll
@@ -618,7 +619,7 @@ __device__ __forceinline__ void stage_catt(const Params& p, const MCtx& c, int p
   // O^T / l as operand fragments (see pi05_bs1.hip)
   const float inv = lsum > 0.f ? 1.0f / lsum : 0.f;
   const bool odd = c.lq & 1;
-  const uint32_t ob = c.xb + K::X_CP + (uint32_t)((c.r * NCW + c.wave) * K::NI * 3072 + (c.lr * 4 + (c.lq >> 1) + 2 * (c.lq & 1)) * 16);
+  const uint32_t ob = c.xb + K::X_CP + (uint32_t)((c.r * NCW + c.wave) * K::NI * 3072 + (((c.lq >> 1) + 2 * (c.lq & 1)) * 16 + c.lr) * 16);
 #pragma unroll
   for (int ks = 0; ks < 3; ks++) {
     const unsigned a0 = pack_bf16x2(o[2 * ks][0] * inv, o[2 * ks][1] * inv);
@@ -639,7 +640,7 @@ template <class K>
 __device__ __forceinline__ void stage_comb(const Params& p, const Ctx& c) {
   constexpr int TT = K::TT;
   if (c.r >= 3 * K::HX) return;
-  const int hh = c.r / 3, ks = c.r - 3 * hh, tt = tile_of<K>(c), t = 16 * tt + (c.lane >> 2);
+  const int hh = c.r / 3, ks = c.r - 3 * hh, tt = tile_of<K>(c), t = 16 * tt + c.lr;
   const bool tv = t < p.Tv;
 #pragma unroll
   for (int i = 0; i < K::NI; i++) {
@@ -652,7 +653,7 @@ __device__ __forceinline__ void stage_comb(const Params& p, const Ctx& c) {
 #pragma unroll
     for (int q = 0; q < K::NCH; q++) {
       const int rw = (r0 + q / K::NP) * NCW + tt + 2 * (q % K::NP);
-      ml[q] = ldb64<kCpSc1>(c.ws, tv ? c.xb + K::X_CML + (uint32_t)(rw * K::NI * 128 + (c.lane >> 2) * 8) : OOB);
+      ml[q] = ldb64<kCpSc1>(c.ws, tv ? c.xb + K::X_CML + (uint32_t)(rw * K::NI * 128 + c.lr * 8) : OOB);
       v[q] = ldb128<kCpSc1>(c.ws, tv ? c.xb + K::X_CP + (uint32_t)(rw * K::NI * 3072 + ks * 1024 + c.lane * 16) : OOB);
     }
     __builtin_amdgcn_sched_barrier(0);

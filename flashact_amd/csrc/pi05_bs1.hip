@@ -245,8 +245,7 @@ __device__ __forceinline__ void page_release(const Ctx& c, int upto) {
 }
 
 __device__ __forceinline__ void dma16(const void* g, uint32_t lds_addr) {
-  // global_load_lds_dwordx4: lane i copies 16 bytes from g to LDS m0 + 16 i, so a fragment lands
-  // in MFMA lane order. Inline asm keeps the compiler from draining these copies at waits it
+  // global_load_lds_dwordx4: lane i copies 16 bytes from g to LDS m0 + 16 i. Inline asm keeps the compiler from draining these copies at waits it
   // inserts for other memory operations; m0 is saved and restored (the compiler reserves it).
   unsigned saved;
   asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
@@ -260,7 +259,8 @@ __device__ __forceinline__ int qkv_row(int g, int vr) {
 }
 
 // Pages of one layer (i = page index within the layer). Loader wave lw copies fragments
-// 8lw..8lw+7 of each page; fragment f lands at ring slot offset f*1024 in MFMA lane order.
+// 8lw..8lw+7 of each page; fragment f lands at ring slot offset f*1024, its rows and 16-byte chunks in
+// the order of copy_row / copy_chunk (below, lr and lq are the row and the chunk).
 //   0-3 QKV  (fragment F = 16i + f: row tile F/32, k-step F%32; 24 rows, tile 1 holds 8)
 //   4   K    (F: key tile F/8, k-step F%8) of keys kb0..kb0+31 (rows past the prefix: key 0)
 //   5   V^T  (F: dim tile; lane (lr, lq) holds keys kb0 + 8lq .. +8 of dim 16F + lr)
@@ -281,6 +281,7 @@ struct LoaderBases {
 template <bool FP8>
 __device__ __forceinline__ void loader_bases(const Params& p, const Ctx& c, int lw, LoaderBases& L) {
   using P = Pages<FP8>;
+  const int cr = copy_row(c.lane), cq = copy_chunk(c.lane);
   const unsigned char* w1 = reinterpret_cast<const unsigned char*>(p.w1);
   const unsigned char* wo = reinterpret_cast<const unsigned char*>(p.wo);
   const unsigned char* w2 = reinterpret_cast<const unsigned char*>(p.w2);
@@ -288,41 +289,41 @@ __device__ __forceinline__ void loader_bases(const Params& p, const Ctx& c, int 
   if constexpr (FP8) {
 #pragma unroll
     for (int i = 0; i < P::NQKV; i++) {
-      const int lr = (i == 1 && c.lr >= 8) ? c.lr - 8 : c.lr;
-      L.b[P::QKV + i] = w1 + (size_t)qkv_row(c.g, 24 * c.r + i * 16 + lr) * D + 512 * lw + 16 * c.lq;
+      const int lr = (i == 1 && cr >= 8) ? cr - 8 : cr;
+      L.b[P::QKV + i] = w1 + (size_t)qkv_row(c.g, 24 * c.r + i * 16 + lr) * D + 512 * lw + 16 * cq;
     }
-    L.b[P::O] = wo + (size_t)(32 * c.r + 16 * lw + c.lr) * 2048 + 256 * c.g + 16 * c.lq;
+    L.b[P::O] = wo + (size_t)(32 * c.r + 16 * lw + cr) * 2048 + 256 * c.g + 16 * cq;
 #pragma unroll
     for (int i = 0; i < P::NGU; i++)
-      L.b[P::GU + i] = w2 + (size_t)(1024 * c.g + 32 * c.r + 16 * i + c.lr) * D + 512 * lw + 16 * c.lq;
-    L.b[P::DN] = w3 + (size_t)(32 * c.r + 16 * lw + c.lr) * 4096 + 512 * c.g + 16 * c.lq;
+      L.b[P::GU + i] = w2 + (size_t)(1024 * c.g + 32 * c.r + 16 * i + cr) * D + 512 * lw + 16 * cq;
+    L.b[P::DN] = w3 + (size_t)(32 * c.r + 16 * lw + cr) * 4096 + 512 * c.g + 16 * cq;
   } else {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const int F0 = 16 * i + 8 * lw, rt = F0 >> 5, ks0 = F0 & 31;
-      const int lr = (rt == 1 && c.lr >= 8) ? c.lr - 8 : c.lr;
-      L.b[i] = w1 + ((size_t)qkv_row(c.g, 24 * c.r + rt * 16 + lr) * D + ks0 * 32 + c.lq * 8) * 2;
+      const int lr = (rt == 1 && cr >= 8) ? cr - 8 : cr;
+      L.b[i] = w1 + ((size_t)qkv_row(c.g, 24 * c.r + rt * 16 + lr) * D + ks0 * 32 + cq * 8) * 2;
     }
-    L.b[P::O] = wo + ((size_t)(32 * c.r + 16 * lw + c.lr) * 2048 + 256 * c.g + c.lq * 8) * 2;
+    L.b[P::O] = wo + ((size_t)(32 * c.r + 16 * lw + cr) * 2048 + 256 * c.g + cq * 8) * 2;
 #pragma unroll
     for (int i = P::GU; i < P::DN; i++) {
       const int F0 = 16 * (i - P::GU) + 8 * lw, rt = F0 >> 5, ks0 = F0 & 31;
-      L.b[i] = w2 + ((size_t)(1024 * c.g + 32 * c.r + 16 * rt + c.lr) * D + ks0 * 32 + c.lq * 8) * 2;
+      L.b[i] = w2 + ((size_t)(1024 * c.g + 32 * c.r + 16 * rt + cr) * D + ks0 * 32 + cq * 8) * 2;
     }
 #pragma unroll
     for (int i = P::DN; i < P::PPL; i++)
-      L.b[i] = w3 + ((size_t)(32 * c.r + 16 * (i - P::DN) + c.lr) * 4096 + 512 * c.g + 8 * lw * 32 + c.lq * 8) * 2;
+      L.b[i] = w3 + ((size_t)(32 * c.r + 16 * (i - P::DN) + cr) * 4096 + 512 * c.g + 8 * lw * 32 + cq * 8) * 2;
   }
   {
-    int key = c.kb0 + 16 * lw + c.lr;
+    int key = c.kb0 + 16 * lw + cr;
     if (key >= p.Lp) key = 0;
-    L.b[P::K] = reinterpret_cast<const unsigned char*>(p.kcache + (size_t)key * HD + c.lq * 8);
+    L.b[P::K] = reinterpret_cast<const unsigned char*>(p.kcache + (size_t)key * HD + cq * 8);
     // An 8-key group that starts inside the prefix is copied from its own row even when it runs
     // past Lp (it stays inside the row: Lmax >= 8 * ceil(Lp / 8)); keys >= Lp are masked by the
     // attention stage. Groups entirely past the prefix copy keys 0..7 instead.
-    int kv = c.kb0 + 8 * c.lq;
+    int kv = c.kb0 + 8 * cq;
     if (kv >= p.Lp) kv = 0;
-    L.b[P::V] = reinterpret_cast<const unsigned char*>(p.vtcache + (size_t)(128 * lw + c.lr) * p.Lmax + kv);
+    L.b[P::V] = reinterpret_cast<const unsigned char*>(p.vtcache + (size_t)(128 * lw + cr) * p.Lmax + kv);
   }
 }
 
@@ -449,8 +450,8 @@ __device__ __forceinline__ f32x4 mfma_kv(u32x4 a, u32x4 b, f32x4 c) {
 
 // acc[rt] = sum_k W[row tile rt][k] * X[token 16w+lr][k] over KS k-steps. bf16 weights: fragment
 // F = rt*KS + ks is slot F%16 of ring page pg0 + F/16. fp8 weights: pair P = rt*PRT + ks/2 is slot
-// P%16 of page pg0 + P/16; its 1 KB holds row lr, k 16q..16q+15 of the pair at byte 16 (lr + 16 q),
-// so k-step ks reads 8 bytes at 16 lr + 256 (2 (ks%2) + lq/2) + 8 (lq%2). xoff = byte offset in the
+// P%16 of page pg0 + P/16; its 1 KB holds row lr, k 16q..16q+15 of the pair at frag_slot(lr, q),
+// so k-step ks reads 8 bytes at frag_slot(lr, 2 (ks%2) + lq/2) + 8 (lq%2). xoff = byte offset in the
 // workspace of X[token][k = 8 lq] (OOB for tokens >= Tv: the loads return zeros); k-step ks adds
 // XSTRIDE bytes.
 struct NoWait {
@@ -476,7 +477,7 @@ __device__ __forceinline__ void gemm_tok(f32x4 (&acc)[RT], const Ctx& c, int pg0
   page_wait(c, pg0 + NPG - 1);
   stamp(c, ts);
   uint32_t slot[NPG];
-  const uint32_t loff = FP8 ? 16 * c.lr + 256 * (c.lq >> 1) + 8 * (c.lq & 1) : c.lane * 16;
+  const uint32_t loff = FP8 ? frag_slot(c.lr, c.lq >> 1) + 8 * (c.lq & 1) : frag_slot(c.lr, c.lq);
 #pragma unroll
   for (int k = 0; k < NPG; k++) slot[k] = ((pg0 + k) % RING) * PAGE + loff;
 #pragma unroll
@@ -498,7 +499,7 @@ __device__ __forceinline__ void gemm_tok(f32x4 (&acc)[RT], const Ctx& c, int pg0
         const int k = (h + j) / RT, rt = (h + j) % RT;
         if constexpr (FP8) {
           const int ks = ck * KC + k, P = rt * PRT + (ks >> 1);
-          const u32x2 q = *reinterpret_cast<const u32x2*>(fa_lds + slot[P >> 4] + (P & 15) * 1024 + 512 * (ks & 1));
+          const u32x2 q = *reinterpret_cast<const u32x2*>(fa_lds + (slot[P >> 4] ^ (32u * (ks & 1))) + (P & 15) * 1024);
           af[j] = fp8x8_to_bf16(q[0], q[1]);
         } else {
           const int F = rt * KS + ck * KC + k;
@@ -833,7 +834,7 @@ __device__ __forceinline__ void stage_att(const Params& p, const Ctx& c, int l, 
       if constexpr (first) {  // the ring page
 #pragma unroll
         for (int ks = 0; ks < 8; ks++)
-          kf[ks] = *reinterpret_cast<const u32x4*>(fa_lds + kslot + (kt * 8 + ks) * 1024 + c.lane * 16);
+          kf[ks] = *reinterpret_cast<const u32x4*>(fa_lds + kslot + (kt * 8 + ks) * 1024 + frag_slot(c.lr, c.lq));
       } else {
         const uint32_t rb = key < kend ? kl + key * HD * 2 + c.lq * 16 : OOB;
 #pragma unroll
@@ -895,7 +896,7 @@ __device__ __forceinline__ void stage_att(const Params& p, const Ctx& c, int l, 
         const int kg = kg0 + 16 * h2;
         if constexpr (first) {  // the ring page
           const int o8 = 16 * h2 + 4 * c.lq;  // key offset within the 32-key block
-          const uint32_t ad = vslot + (c.lr + 16 * (o8 >> 3)) * 16 + (o8 & 7) * 2 + half * 8 * 1024;
+          const uint32_t ad = vslot + frag_slot(c.lr, o8 >> 3) + (o8 & 7) * 2 + half * 8 * 1024;
 #pragma unroll
           for (int d8 = 0; d8 < 8; d8++) vf[d8][h2] = *reinterpret_cast<const u32x2*>(fa_lds + ad + d8 * 1024);
         } else {

@@ -82,7 +82,7 @@ struct Cfg {
   static_assert(NB * HX * NKC == NR && NKC >= 2 && NB <= 2, "one attention item per rank");
 };
 __host__ __device__ constexpr uint32_t frag_off(int KS, int t, int k) {  // as in pi05_bs1.hip
-  return (uint32_t)(((((t >> 4) * KS + (k >> 5)) * 16 + (t & 15)) * 4 + ((k >> 3) & 3)) * 16 + (k & 7) * 2);
+  return (uint32_t)(((((t >> 4) * KS + (k >> 5)) * 4 + ((k >> 3) & 3)) * 16 + (t & 15)) * 16 + (k & 7) * 2);
 }
 
 struct Params {
@@ -129,7 +129,8 @@ struct Loader : LoaderBase<K> {
 
   __device__ void run() {
     const int NL = p.NL;
-    const uint32_t vq = c.lr * (D * 2) + c.lq * 16, vo = c.lr * (QD * 2) + c.lq * 16, vd = c.lr * (FF * 2) + c.lq * 16;
+    const int cr = copy_row(c.lane), cq = copy_chunk(c.lane);
+    const uint32_t vq = cr * (D * 2) + cq * 16, vo = cr * (QD * 2) + cq * 16, vd = cr * (FF * 2) + cq * 16;
     const int win = c.r / (NR / K::C), rg = c.r % (NR / K::C);  // K window and row group of O and down
     const int b = c.grp + c.an * K::NGRP;
     const uint32_t vstep = 16u * p.Lmax * 2;
@@ -147,19 +148,19 @@ struct Loader : LoaderBase<K> {
 #pragma unroll 1
         for (int i = 0; i < np; i++) {  // K: key tile this->lw, k-step f; keys past the chunk copy key 0 (masked later)
           if (!this->room()) break;
-          int key = c.kbeg + 64 * u0 + 32 * i + 8 * (c.lr >> 2) + 4 * this->lw + (c.lr & 3);
+          int key = c.kbeg + 64 * u0 + 32 * i + 8 * (cr >> 2) + 4 * this->lw + (cr & 3);
           if (key >= c.kend) key = 0;
           const uint32_t d = this->dst();
 #pragma unroll
-          for (int f = 0; f < 8; f++) dma16(kb + f * 64, (uint32_t)key * (HD * 2) + c.lq * 16, d + f * 1024);
+          for (int f = 0; f < 8; f++) dma16(kb + f * 64, (uint32_t)key * (HD * 2) + cq * 16, d + f * 1024);
           this->pg++;
         }
 #pragma unroll 1
         for (int i = 0; i < np; i++) {  // V^T: dim tile 8 this->lw + f; an 8-key group that starts in the chunk
           if (!this->room()) break;         // stays within the row (Lmax)
-          int kv = c.kbeg + 64 * u0 + 32 * i + 8 * c.lq;
+          int kv = c.kbeg + 64 * u0 + 32 * i + 8 * cq;
           if (kv >= c.kend) kv = 0;
-          const uint32_t vv = (uint32_t)c.lr * p.Lmax * 2 + kv * 2;
+          const uint32_t vv = (uint32_t)cr * p.Lmax * 2 + kv * 2;
           const uint32_t d = this->dst();
 #pragma unroll
           for (int f = 0; f < 8; f++) dma16(vb + (size_t)(8 * this->lw + f) * vstep, vv, d + f * 1024);
@@ -188,7 +189,7 @@ __device__ __forceinline__ void tok_off(const Params& p, const PCtx& c, uint32_t
   const int t = 16 * c.wave + c.lr;
 #pragma unroll
   for (int n = 0; n < K::NB; n++)
-    o[n] = t < p.Tv && n < c.ns ? c.xb + base + (uint32_t)(((n * 4 + c.wave) * KT + ks0) * 1024 + (c.lr * 4 + c.lq) * 16) : OOB;
+    o[n] = t < p.Tv && n < c.ns ? c.xb + base + (uint32_t)(((n * 4 + c.wave) * KT + ks0) * 1024 + c.lane * 16) : OOB;
 }
 
 // ---------------------------------------------------------------- norm stages
@@ -489,7 +490,7 @@ __device__ __forceinline__ void stage_att(const Params& p, const PCtx& c, int li
       page_wait<K>(c, pk + 2 * u + 1);
       u32x4 kf[2][8];
       auto rd = [&](int q) {
-        const uint32_t a = ((pk + 2 * u + (q >> 1)) % RING) * PAGE + c.lane * 16 + (q & 1) * 8192;
+        const uint32_t a = ((pk + 2 * u + (q >> 1)) % RING) * PAGE + frag_slot(c.lr, c.lq) + (q & 1) * 8192;
 #pragma unroll
         for (int ks = 0; ks < 8; ks++) kf[q & 1][ks] = *reinterpret_cast<const u32x4*>(fg_lds + a + ks * 1024);
       };
@@ -517,7 +518,7 @@ __device__ __forceinline__ void stage_att(const Params& p, const PCtx& c, int li
       page_wait<K>(c, pv + 2 * u + 1);
       u32x4 vf[2][8];
       auto rd = [&](int q) {  // half q & 1 of the dims of block q / 2
-        const uint32_t a = ((pv + 2 * u + (q >> 1)) % RING) * PAGE + c.lane * 16 + (q & 1) * 8192;
+        const uint32_t a = ((pv + 2 * u + (q >> 1)) % RING) * PAGE + frag_slot(c.lr, c.lq) + (q & 1) * 8192;
 #pragma unroll
         for (int d8 = 0; d8 < 8; d8++) vf[q & 1][d8] = *reinterpret_cast<const u32x4*>(fg_lds + a + d8 * 1024);
       };
@@ -542,7 +543,7 @@ __device__ __forceinline__ void stage_att(const Params& p, const PCtx& c, int li
   // O^T / l in the O projection's operand order, whole 16-byte slots (see pi05_bs1.hip)
   const float inv = lsum > 0.f ? 1.0f / lsum : 0.f;
   const bool odd = c.lq & 1;
-  const uint32_t ob = c.xb + K::X_ATTP + (uint32_t)((c.r * 4 + c.wave) * 8192 + (c.lr * 4 + (c.lq >> 1) + 2 * (c.lq & 1)) * 16);
+  const uint32_t ob = c.xb + K::X_ATTP + (uint32_t)((c.r * 4 + c.wave) * 8192 + (((c.lq >> 1) + 2 * (c.lq & 1)) * 16 + c.lr) * 16);
 #pragma unroll
   for (int ks = 0; ks < 8; ks++) {
     const unsigned a0 = pack_bf16x2(o[2 * ks][0] * inv, o[2 * ks][1] * inv);
@@ -567,7 +568,7 @@ __device__ __forceinline__ void stage_comb(const Params& p, const PCtx& c) {
   const int nh = id0 >> 3, n = nh / K::HX;  // a rank's ids share their (slot, head)
   if (n >= c.ns) return;
   xcd_wait(c, (K::NKC == 32 ? 0xffffffffu : ((1u << (K::NKC & 31)) - 1u)) << (nh * K::NKC));
-  const int t = 16 * c.wave + (c.lane >> 2);
+  const int t = 16 * c.wave + c.lr;
   const bool tv = t < p.Tv;
   u32x2 ml[K::NKC];
   u32x4 v[NF][K::NKC];
