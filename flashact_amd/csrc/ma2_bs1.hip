@@ -19,8 +19,8 @@
 //          -> h = silu(g + b_g) (u + b_u)                                                       [X]
 //   DN     all ranks: 24 rows of W_dn[:, 384g..384g+384) x h_g -> partial                      {E}
 // (the reference runs every stage behind a grid-wide barrier: src/molmoact2/mk_ma2.cu:286-561).
-// Weight fragments of the next GEMM stage (and the context K/V of the attention stage) are loaded
-// into registers before each wait, so HBM latency overlaps the synchronisation.
+// The large weights of a layer are copied to LDS in windows where most waves only wait (copy_gu); the SO and
+// CO weights and the context K/V are loaded into registers before a wait, so HBM latency overlaps it.
 // GEMMs: v_mfma_f32_16x16x32_bf16 with 16 weight rows as A and 16 tokens as B; activations are
 // kept in MFMA fragment order in each XCD's L2 (plain stores, sc1 loads).
 #include "engine.h"
@@ -70,7 +70,13 @@ constexpr uint32_t L_X = L_RED + 16 * 1024;         // residual x of token r [76
 constexpr uint32_t L_XT = L_X + D * 4;              // x_t of token r [32] f32
 constexpr uint32_t L_MISC = L_XT + AD * 4;          // [4 waves][768] f32 exchange partial sums
 constexpr uint32_t L_ROPE = L_MISC + 4 * D * 4;     // rank 0: RoPE cos | sin [2][32 tokens][48] f32
-constexpr uint32_t LDS_BYTES = L_ROPE + 2 * TP * 48 * 4;
+constexpr uint32_t L_GU = L_ROPE + 2 * TP * 48 * 4;  // gate/up weights of the layer [4 waves][2 row tiles][6 k-steps][1 KB]
+constexpr uint32_t L_DN = L_GU + 48 * 1024;         // down weights [2 row tiles][12 k-steps][1 KB]
+constexpr uint32_t L_QKV = L_ATT + 12 * 1024;  // next layer's QKV weights [24 k-steps][1 KB], from the cross attention
+                                               // (whose q takes the 12 KB below) to the QKV stage
+constexpr uint32_t L_CQ = L_DN;    // CQ weights [24 k-steps][1 KB], from the self attention to the CQ stage
+constexpr uint32_t LDS_BYTES = L_DN + 24 * 1024;
+static_assert(LDS_BYTES <= 160 * 1024, "LDS of one CU");
 
 struct Params {
   const bf16 *w_qkv, *w_so, *w_cq, *w_co, *w_gu, *w_dn;
@@ -127,6 +133,13 @@ __device__ __forceinline__ bool aborted(const Ctx& c) {
 // workgroup barrier): 11.48-11.55 -> 11.15-11.17 ms per chunk.
 __device__ __forceinline__ void xarrive(Ctx& c) {
   __builtin_amdgcn_s_waitcnt(0);  // this wave's global and LDS operations are complete
+  c.e += 1;
+  if (c.lane == 0) __hip_atomic_store(c.xflag + c.r * 4 + c.w, c.e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// As xarrive for a wave whose outstanding memory operations are weight copies to LDS alone: they land under
+// the wait (this wave drains them at its next xarrive, before any wave reads them).
+__device__ __forceinline__ void xarrive_copies(Ctx& c) {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   c.e += 1;
   if (c.lane == 0) __hip_atomic_store(c.xflag + c.r * 4 + c.w, c.e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
@@ -282,20 +295,22 @@ __device__ __forceinline__ void stage_norm(const Params& p, const Ctx& c, int bu
 
 // ---- GEMM pieces -------------------------------------------------------------------------------
 // One 16-row weight tile over all 32 tokens, K = 768 split over the 4 waves (k-steps 6w..6w+5;
-// wf = this wave's weight fragments, loaded ahead). The four partial sums meet in LDS; waves 0/1
+// weights in LDS at wl). The four partial sums meet in LDS; waves 0/1
 // finish token tiles 0/1: + bias, columns col0 + 4 lq .. + 3 (of ns 96-column parts) into the
 // lane-major layout of X_QKV / X_QC at `out` (each store instruction writes 4 runs of 256 bytes;
 // row-major [token][column] rows read back by lanes 96 bytes apart took the self attention's loads
 // through about seven 128-byte lines per kilobyte used).
-__device__ __forceinline__ void gemm16(const Params& p, const Ctx& c, const u32x4 (&wf)[6], uint32_t out, int ns,
-                                       int col0, const float* bias) {
+__device__ __forceinline__ void gemm16(const Params& p, const Ctx& c, uint32_t wl, uint32_t out, int ns, int col0,
+                                       const float* bias) {
   f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-  u32x4 b[2][6];
+  u32x4 b[2][6], wf[6];
 #pragma unroll
   for (int j = 0; j < 6; j++)
 #pragma unroll
     for (int tt = 0; tt < 2; tt++)
       b[tt][j] = ldb128<kCpSc1>(c.ws, c.xb + X_XN + (uint32_t)(((tt * (D / 32) + 6 * c.w + j) * 64 + c.lane) * 16));
+#pragma unroll
+  for (int j = 0; j < 6; j++) wf[j] = lds128(wl + (6 * c.w + j) * 1024 + frag_slot(c.lr, c.lq));
 #pragma unroll
   for (int j = 0; j < 6; j++)
 #pragma unroll
@@ -322,8 +337,8 @@ __device__ __forceinline__ int row24(int base, int rt, int lr) { return base + 1
 // Partial-sum projection of this XCD's K-window onto 24 output rows (SO / CO: K = 96 over the
 // head's attention output; DN: K = 384 over h). Wave w = (row tile w / 2, token tile w % 2); the
 // tagged fp32 partial goes to exchange buffer `buf` with the parity bit `par`.
-template <int NK>
-__device__ __forceinline__ void proj24(const Params& p, const Ctx& c, const u32x4 (&wf)[NK], uint32_t act, int KS,
+template <int NK, class WF>
+__device__ __forceinline__ void proj24(const Params& p, const Ctx& c, const WF& wf, uint32_t act, int KS,
                                        int buf, unsigned par) {
   const int rt = c.w >> 1, tt = c.w & 1;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -331,7 +346,7 @@ __device__ __forceinline__ void proj24(const Params& p, const Ctx& c, const u32x
 #pragma unroll
   for (int j = 0; j < NK; j++) b[j] = ldb128<kCpSc1>(c.ws, c.xb + act + (uint32_t)(((tt * KS + j) * 64 + c.lane) * 16));
 #pragma unroll
-  for (int j = 0; j < NK; j++) acc = mfma16(wf[j], b[j], acc);
+  for (int j = 0; j < NK; j++) acc = mfma16(wf(j), b[j], acc);
   const int t = 16 * tt + c.lr;
   // Every token slot is written (zeros past Tv): a slot left over from an earlier launch with a
   // larger Tv could otherwise carry the parity this launch waits for.
@@ -544,16 +559,20 @@ __device__ __forceinline__ void stage_comb(const Params& p, const Ctx& c) {
   }
 }
 
-// gate/up rows 24r.. of the head's slice: K = 768 split over the waves (wf[rt][j] = k-step 6w + j)
+// gate/up rows 24r.. of the head's slice: K = 768 split over the waves (weights in LDS: k-step 6w + j)
 // -> LDS -> wave (rt, tt) adds, applies biases and silu(g) u, stores h_g fragments.
-__device__ __forceinline__ void stage_gu(const Params& p, const Ctx& c, const u32x4 (&wf)[2][6], const float* bias) {
+__device__ __forceinline__ void stage_gu(const Params& p, const Ctx& c, const float* bias) {
   f32x4 acc[2][2] = {};
-  u32x4 b[2][6];
+  u32x4 b[2][6], wf[2][6];
 #pragma unroll
   for (int j = 0; j < 6; j++)
 #pragma unroll
     for (int tt = 0; tt < 2; tt++)
       b[tt][j] = ldb128<kCpSc1>(c.ws, c.xb + X_XN + (uint32_t)(((tt * (D / 32) + 6 * c.w + j) * 64 + c.lane) * 16));
+#pragma unroll
+  for (int rt = 0; rt < 2; rt++)
+#pragma unroll
+    for (int j = 0; j < 6; j++) wf[rt][j] = lds128(L_GU + ((c.w * 2 + rt) * 6 + j) * 1024 + frag_slot(c.lr, c.lq));
 #pragma unroll
   for (int j = 0; j < 6; j++)
 #pragma unroll
@@ -577,6 +596,47 @@ __device__ __forceinline__ void stage_gu(const Params& p, const Ctx& c, const u3
       pack_bf16x2(silu(sm[0]) * sm[1], silu(sm[2]) * sm[3]);
 }
 
+// Weight copies to LDS, fragment by fragment (see copy_row), by waves that would only wait, and long before
+// their use: gate/up (48) and CQ (24) by waves 2 and 3 during the self attention, the next layer's QKV (24)
+// by waves 2 and 3 during the cross attention, down (24) by waves 1-3 during the combine. Loaded into
+// registers in MFMA lane order just ahead of the norms' exchanges and the down stage's barrier instead (the
+// address unit takes such a load lane by lane, 64 clocks per kilobyte), they stood in line before those
+// waits' polls. Per layer at Lk = 493: N_mlp 4.1 -> 2.1 us, DN 1.9 -> 0.9, N_msa 3.0 -> 2.4, N_mca 3.5 -> 2.5;
+// a chunk 10.90 -> 9.59 ms (gate/up and down alone 9.90), at Lk = 777 11.19 -> 9.71. QKV copied in the
+// combine's window delayed the combine's own loads (9.69); rank 0's gate/up copies held back until its
+// self attention has stored cost more at the barrier after it than they gave there (9.72).
+__device__ __forceinline__ void copy_gu(const Params& p, const Ctx& c, int l) {
+  const bf16* W = p.w_gu + (size_t)l * GUN * D + 8 * copy_chunk(c.lane);
+  const bf16* r0 = W + (size_t)(2 * 384 * c.g + row24(24 * c.r, 0, copy_row(c.lane))) * D;
+  const bf16* r1 = W + (size_t)(2 * 384 * c.g + row24(24 * c.r, 1, copy_row(c.lane))) * D;
+#pragma unroll
+  for (int q = 0; q < 24; q++) {  // fragment (wave w2, row tile rt, k-step j) of this wave's half
+    const int w2 = 2 * (c.w & 1) + q / 12, rt = (q / 6) & 1, j = q % 6;
+    dma16<false>((rt ? r1 : r0) + 32 * (6 * w2 + j), lds_addr(L_GU + ((w2 * 2 + rt) * 6 + j) * 1024));
+  }
+}
+// 16 weight rows x 768 to LDS [4 waves][6 k-steps][1 KB], by waves W0..3.
+template <int W0>
+__device__ __forceinline__ void copy16(const Ctx& c, const bf16* W, int row, uint32_t dst) {
+  const bf16* r = W + (size_t)(row + copy_row(c.lane)) * D + 8 * copy_chunk(c.lane);
+  constexpr int N = 24 / (4 - W0);
+#pragma unroll
+  for (int q = 0; q < N; q++) {
+    const int f = N * (c.w - W0) + q;
+    dma16<false>(r + 32 * f, lds_addr(dst + f * 1024));
+  }
+}
+__device__ __forceinline__ void copy_dn(const Params& p, const Ctx& c, int l) {
+  const bf16* W = p.w_dn + (size_t)l * D * FF + 384 * c.g + 8 * copy_chunk(c.lane);
+  const bf16* r0 = W + (size_t)row24(24 * c.r, 0, copy_row(c.lane)) * FF;
+  const bf16* r1 = W + (size_t)row24(24 * c.r, 1, copy_row(c.lane)) * FF;
+#pragma unroll
+  for (int q = 0; q < 8; q++) {
+    const int f = 8 * (c.w - 1) + q;  // row tile f / 12, k-step f % 12
+    dma16<false>((f >= 12 ? r1 : r0) + 32 * (f >= 12 ? f - 12 : f), lds_addr(L_DN + f * 1024));
+  }
+}
+
 // ---- the kernel --------------------------------------------------------------------------------
 __device__ __forceinline__ void mark(const Params& p, int idx, uint64_t& t0) {
   if (p.stage_cycles && blockIdx.x == 0 && threadIdx.x == 0) {
@@ -586,7 +646,7 @@ __device__ __forceinline__ void mark(const Params& p, int idx, uint64_t& t0) {
   }
 }
 
-// NC: context chunk slots of the combine, 16 (Lk <= 512: 10.9 ms per chunk at Lk = 493) or 32 (11.16 ms
+// NC: context chunk slots of the combine, 16 (Lk <= 512: 9.59 ms per chunk at Lk = 493) or 32 (9.71 ms
 // at Lk = 777, which took 27.6 ms on the stage-engine kernel).
 template <int NC>
 __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
@@ -637,6 +697,11 @@ __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
   auto buf = [](int e) { return e & 1; };
   auto par = [&](int e) { return (1u + ((e & 1) ? base1 : base0) + (unsigned)(e >> 1)) & 1u; };
   const int NL = p.NL;
+  auto copy_qkv = [&](int l) {  // waves 2 and 3: the QKV weights of ranks 0..17
+    if (c.r < 18)
+      copy16<2>(c, p.w_qkv + (size_t)l * QKVN * D, (c.r / 6) * D + HD * c.g + 16 * (c.r % 6), L_QKV);
+  };
+  if (c.w >= 2) copy_qkv(0);
   const float dt = 1.0f / (float)p.S;
   uint64_t t0 = __builtin_amdgcn_s_memrealtime();
 #pragma unroll 1
@@ -647,14 +712,7 @@ __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
       const int li = step * NL + l;
       const float* mo = p.mods + ((size_t)step * NL + l) * 9 * D;
       const int e0 = 3 * li, e1 = e0 + 1, e2 = e0 + 2;
-      // N_msa, with the QKV weights of ranks 0..17 in flight
-      u32x4 wq[6];
-      if (c.r < 18) {
-        const int row = (c.r / 6) * D + HD * c.g + 16 * (c.r % 6) + c.lr;
-        const bf16* W = p.w_qkv + (size_t)l * QKVN * D;
-#pragma unroll
-        for (int j = 0; j < 6; j++) wq[j] = wfrag(W, D, row, 32 * (6 * c.w + j), c.lq);
-      }
+      // N_msa
       if (l == 0)
         stage_norm<0>(p, c, 0, 0u, nullptr, nullptr, mo, mo + D, 0.f);
       else
@@ -666,7 +724,7 @@ __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
       mark(p, 15, t0);
       // QKV
       if (c.r < 18)
-        gemm16(p, c, wq, X_QKV, 3, 96 * (c.r / 6) + 16 * (c.r % 6),
+        gemm16(p, c, L_QKV, X_QKV, 3, 96 * (c.r / 6) + 16 * (c.r % 6),
                p.b_qkv + (size_t)l * QKVN + (c.r / 6) * D + HD * c.g + 16 * (c.r % 6));
       mark(p, 1, t0);
       xarrive(c);
@@ -682,20 +740,21 @@ __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
       // SATT
       if (c.r == 0) stage_satt(p, c);
       mark(p, 2, t0);
-      xarrive(c);
+      static_assert(TP <= 32, "waves 2 and 3 hold no token of the self attention");
+      if (c.w >= 2) {
+        copy_gu(p, c, l);
+        if (c.r < 6) copy16<2>(c, p.w_cq + (size_t)l * D * D, HD * c.g + 16 * c.r, L_CQ);
+        xarrive_copies(c);
+      } else {
+        xarrive(c);
+      }
       xwait(c);
       mark(p, 15, t0);
       // SO -> exchange e0
-      proj24<3>(p, c, wso, X_ATT, 3, buf(e0), par(e0));
+      proj24<3>(p, c, [&](int j) { return wso[j]; }, X_ATT, 3, buf(e0), par(e0));
       mark(p, 3, t0);
-      // N_mca, with the CQ weights (ranks 0..5) and this rank's context keys/values in flight
-      u32x4 wc[6], kf[2][3], vf[6];
-      if (c.r < 6) {
-        const bf16* W = p.w_cq + (size_t)l * D * D;
-        const int row = HD * c.g + 16 * c.r + c.lr;
-#pragma unroll
-        for (int j = 0; j < 6; j++) wc[j] = wfrag(W, D, row, 32 * (6 * c.w + j), c.lq);
-      }
+      // N_mca, with this rank's context keys/values in flight
+      u32x4 kf[2][3], vf[6];
       if (KPR * c.r < p.Lk && c.w < 2) {
         const bf16* K = p.kctx + (size_t)l * p.Lkmax * D;
         const bf16* V = p.vtctx + (size_t)l * D * p.Lkmax;
@@ -718,7 +777,7 @@ __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
       xwait(c);
       mark(p, 15, t0);
       // CQ
-      if (c.r < 6) gemm16(p, c, wc, X_QC, 1, 16 * c.r, p.b_cq + (size_t)l * D + HD * c.g + 16 * c.r);
+      if (c.r < 6) gemm16(p, c, L_CQ, X_QC, 1, 16 * c.r, p.b_cq + (size_t)l * D + HD * c.g + 16 * c.r);
       mark(p, 5, t0);
       xarrive(c);
       xwait(c);
@@ -726,13 +785,23 @@ __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
       // CATT
       stage_catt(p, c, kf, vf);
       mark(p, 6, t0);
-      xarrive(c);
+      if (c.w >= 2) {  // these waves hold no token here either
+        copy_qkv(l + 1 < NL ? l + 1 : 0);
+        xarrive_copies(c);
+      } else {
+        xarrive(c);
+      }
       xwait(c);
       mark(p, 15, t0);
       // COMB, with the CO weights in flight
       stage_comb<NC>(p, c);
       mark(p, 7, t0);
-      xarrive(c);
+      if (c.w > 0) {
+        copy_dn(p, c, l);
+        xarrive_copies(c);
+      } else {
+        xarrive(c);
+      }
       u32x4 wco[3];
       {
         const bf16* W = p.w_co + (size_t)l * D * D;
@@ -743,39 +812,22 @@ __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
       xwait(c);
       mark(p, 15, t0);
       // CO -> exchange e1
-      proj24<3>(p, c, wco, X_ATT, 3, buf(e1), par(e1));
+      proj24<3>(p, c, [&](int j) { return wco[j]; }, X_ATT, 3, buf(e1), par(e1));
       mark(p, 8, t0);
-      // N_mlp, with the gate/up weights in flight
-      u32x4 wg[2][6];
-      {
-        const bf16* W = p.w_gu + (size_t)l * GUN * D;
-#pragma unroll
-        for (int rt = 0; rt < 2; rt++) {
-          const int row = 2 * 384 * c.g + row24(24 * c.r, rt, c.lr);
-#pragma unroll
-          for (int j = 0; j < 6; j++) wg[rt][j] = wfrag(W, D, row, 32 * (6 * c.w + j), c.lq);
-        }
-      }
+      // N_mlp
       stage_norm<1>(p, c, buf(e1), par(e1), p.b_co + (size_t)l * D, mo + 5 * D, mo + 6 * D, mo + 7 * D, 0.f);
       mark(p, 9, t0);
       xarrive(c);
       xwait(c);
       mark(p, 15, t0);
-      // GU, then the down weights in flight
-      stage_gu(p, c, wg, p.b_gu + (size_t)l * GUN + 2 * 384 * c.g);
+      // GU
+      stage_gu(p, c, p.b_gu + (size_t)l * GUN + 2 * 384 * c.g);
       mark(p, 10, t0);
       xarrive(c);
-      u32x4 wd[12];
-      {
-        const bf16* W = p.w_dn + (size_t)l * D * FF;
-        const int row = row24(24 * c.r, c.w >> 1, c.lr);
-#pragma unroll
-        for (int j = 0; j < 12; j++) wd[j] = wfrag(W, FF, row, 384 * c.g + 32 * j, c.lq);
-      }
       xwait(c);
       mark(p, 15, t0);
       // DN -> exchange e2
-      proj24<12>(p, c, wd, X_H, 12, buf(e2), par(e2));
+      proj24<12>(p, c, [&](int j) { return lds128(L_DN + ((c.w >> 1) * 12 + j) * 1024 + frag_slot(c.lr, c.lq)); }, X_H, 12, buf(e2), par(e2));
       mark(p, 11, t0);
     }
     const int el = 3 * (step * NL + NL - 1) + 2;

@@ -57,6 +57,14 @@ def test_ma2_long_context(gpu, Lk, Tv):
     _check(C.make_case(NL=2, Lk=Lk, Tv=Tv, S=2, seed=Lk), gpu)
 
 
+# Batch 1, layer counts whose next layer is the same (1) and an odd one, a single token, a full second token
+# tile and the last row of the first, contexts that leave ranks without keys: the layer's weights lie in LDS
+# regions that other stages and the next layer reuse. Four steps, as for the groups below.
+@pytest.mark.parametrize("NL,Lk,Tv", [(1, 33, 1), (1, 1024, 32), (3, 512, 17), (3, 40, 16)])
+def test_ma2_batch1_layers(gpu, NL, Lk, Tv):
+    _check(C.make_case(NL=NL, Lk=Lk, Tv=Tv, S=4, seed=NL + Lk), gpu)
+
+
 # Every group shape (batch 1-4, 5-8, 9-16, two or four token tiles per sample) with groups of one sample, of
 # none and full, token counts on either side of the tiles, context chunks that are empty, ragged and
 # longer than one softmax segment, and the stage engine past them (17). Four steps: at two, bf16 operands
