@@ -1,6 +1,6 @@
 // MolmoAct2 action-expert flow loop (src/molmoact2/mk_ma2.cu:258-575): the whole S-step Euler
-// loop for a batch of samples in ONE cooperative launch of 256 workgroups x 4 waves, built on the
-// stage engine (engine.h). D = 768, 8 heads of 96, F = 3072, action dim 32 (the first `adim`
+// loop in ONE cooperative launch of 256 workgroups x 4 waves, built on the stage engine (engine.h), for
+// batches past 16 and for shapes or workspaces that ma2_bs1.hip and ma2_group.hip do not take. D = 768, 8 heads of 96, F = 3072, action dim 32 (the first `adim`
 // dims integrated), t_s = s / S, dt = +1/S.
 //
 // Per layer (grid barrier after each stage), token m = b * Tv + t of sample b:

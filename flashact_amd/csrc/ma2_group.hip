@@ -635,7 +635,7 @@ __device__ __forceinline__ void stage_catt(const Params& p, const MCtx& c, int p
 }
 
 // Rank r < 3 HX: head r / 3, k-step r % 3 of it, for the wave's token tiles. A lane owns one 16-byte slot
-// (token lane / 4, 8 dims).
+// (token lane % 16, 8 dims).
 template <class K>
 __device__ __forceinline__ void stage_comb(const Params& p, const Ctx& c) {
   constexpr int TT = K::TT;
@@ -852,7 +852,8 @@ Choice choice() {
   return {(const void*)ma2_group_kernel<G, TT, NB>, Cfg<G, TT, NB>::LDS, Cfg<G, TT, NB>::WS};
 }
 // Wider groups stream fewer weights per XCD but exchange partial sums between XCDs. ms per launch (Lk = 493,
-// Tv = 30, 10 steps), against the stage engine's:
+// Tv = 30, 10 steps), against the stage engine's, all before the copies of copy_row, with which batches 2, 4
+// and 16 run 12.5, 16.4 and 21.5:
 //   batch 2   (4 XCDs, 2 samples) 12.6, (4, 4) 13.7   stage engine 27.6
 //   batch 4   (4, 2) 16.5, (4, 4) 18.3                             28.9
 //   batch 8   (2, 2) 17.7, (4, 4) 21.7                             28.8

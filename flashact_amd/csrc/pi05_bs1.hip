@@ -68,7 +68,7 @@ struct Pages {
   static constexpr int DN = GU + NGU, NDN = FP8 ? 1 : 2, PPL = DN + NDN;
 };
 constexpr int PPL_MAX = Pages<false>::PPL;
-constexpr int MAXF = 1;                                 // pages in flight per loader wave
+constexpr int MAXF = 1;                                 // pages in flight per loader wave (2-7: 1.5-3 % slower)
 constexpr uint32_t OOB = 0x80000000u;                   // buffer offset past every resource
 
 // workspace layout (bytes)
@@ -1320,7 +1320,8 @@ __global__ void __launch_bounds__(NTH, 1) pi05_denoise_bs1(Params p) {
 // Scratch of fa_pi05_denoise_noalloc: one workspace in device memory reserved at load time, so
 // that entry point never allocates. Host code reads its address per device with
 // hipGetSymbolAddress and never uses this name as an address.
-constexpr size_t kNoAllocScratchBytes = size_t(16) << 20;
+// 16 MiB, and the group kernels' flags that every workspace carries: what fitted without them still fits
+constexpr size_t kNoAllocScratchBytes = (size_t(16) << 20) + (kWsDataBase - kWsGroupFlags);
 static_assert(WS_BYTES <= kNoAllocScratchBytes, "the batch-1 workspace fits the static scratch");
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 

@@ -26,7 +26,9 @@
 // What bounds it: each group streams all 34.6 MB of a layer's weights, 34.6/G MB per XCD. The fabric
 // feeds one XCD at 0.85-0.95 TB/s while all eight read (1.0 with four, 1.34 alone): 37 us per layer with
 // G = 1, 19 with G = 2, 10 with G = 4. The stage engine at these batches had 40 to 180 GEMM items for the 256
-// CUs in every stage but gate/up, and eight grid barriers of about 2 us per layer.
+// CUs in every stage but gate/up, and eight grid barriers of about 2 us per layer. At 16 samples a layer takes
+// 88 us: gate/up 20.7, attention 17.5 (its 512 KB of K/V per CU arrive at 44 GB/s; without softmax and P V it
+// takes as long), down 11.1, QKV 8.6, the norms 14.5 with the waits for the partial sums, barriers 5.7.
 #include "group.h"
 #include "../../include/flashact_mi355x.h"
 #include "fa_host.h"
@@ -559,7 +561,7 @@ __device__ __forceinline__ void stage_att(const Params& p, const PCtx& c, int li
 
 // ---------------------------------------------------------------- combine
 // Fragment id = (slot, head, k-step) of token tile w: wave w of rank r takes ids FPR r .. + FPR - 1 (with
-// G = 4: id r of ranks < 16). A lane owns one 16-byte slot (token 16 w + lane / 4, 8 dims).
+// G = 4: id r of ranks < 16). A lane owns one 16-byte slot (token 16 w + lane % 16, 8 dims).
 template <class K>
 __device__ __forceinline__ void stage_comb(const Params& p, const PCtx& c) {
   constexpr int NF = K::FPR > 0 ? K::FPR : 1;
@@ -852,7 +854,8 @@ Choice choice() {
   return {(const void*)pi05_group_kernel<G, NB>, Cfg<G, NB>::LDS, Cfg<G, NB>::WS};
 }
 // Wider groups stream fewer weights per XCD but exchange partial sums between XCDs. Two samples per group
-// share every weight fragment. ms per launch (Lp = 968, Tv = 50, 10 steps), against the stage engine's:
+// share every weight fragment. ms per launch (Lp = 968, Tv = 50, 10 steps), against the stage engine's, all before
+// the copies of copy_row, with which the shapes taken run 5.7, 7.8, 10.3 and 15.9:
 //   batch 2   (4, 1) 6.2, (4, 2) 7.1               stage engine 16.7
 //   batch 4   (4, 2) 8.4, (2, 1) 8.4 (Tv = 10: 6.0 against 6.4)      17.0
 //   batch 8   (2, 2) 11.2, (1, 1) 12.8                               17.4
