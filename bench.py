@@ -45,11 +45,11 @@ TRAFFIC_SOURCE = ("profiles/pi05_denoise_bs1_traffic.md: rocprofv3 --pmc FETCH_S
 PI05_BS1_STAGES = {0: "N1", 1: "QKV", 2: "ATT", 3: "COMB", 4: "O", 5: "N2", 6: "GU", 7: "DN", 8: "FINAL",
                    9: "XCD_waits"}
 PI05_BATCHED_STAGES = {0: "N1", 1: "QKV", 2: "ATT", 3: "COMB", 4: "O", 5: "N2", 6: "GU", 7: "DN", 8: "FINAL",
-                       9: "grid_barriers"}
+                       9: "sync"}
 MA2_BS1_STAGES = {0: "N_msa", 1: "QKV", 2: "SATT", 3: "SO", 4: "N_mca", 5: "CQ", 6: "CATT", 7: "COMB", 8: "CO",
                   9: "N_mlp", 10: "GU", 11: "DN", 12: "FINAL", 15: "XCD_waits"}
 MA2_STAGES = {0: "N_msa", 1: "QKV", 2: "SATT", 3: "SO", 4: "N_mca", 5: "CQ", 6: "CATT", 7: "COMB", 8: "CO",
-              9: "N_mlp", 10: "GU", 11: "GATE_or_GU", 12: "DN", 13: "FINAL", 15: "grid_barriers"}
+              9: "N_mlp", 10: "GU", 11: "GATE_or_GU", 12: "DN", 13: "FINAL", 15: "sync"}
 PREFILL_STAGES = {0: "N1", 1: "QKV", 2: "ATT", 3: "COMB", 4: "O", 5: "N2", 6: "GU", 7: "DN", 9: "grid_barriers"}
 
 
