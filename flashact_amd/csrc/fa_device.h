@@ -43,7 +43,7 @@ constexpr unsigned kSpinCap = 1u << 20;
 // Workspace rules shared by every kernel of the library, so that one workspace may serve any mix
 // of entry points and shapes:
 //  * Bytes [0, kWsDataBase) hold only control words (u64 launch sequence @0, u32 error bits @8,
-//    u32 exchange parity bases @12 and @16, u32 owner @kWsOwner, u32 finished groups @24, zero at
+//    u32 exchange parity (or buffer) bases @12 and @16, u32 owner @kWsOwner, u32 finished groups @24, zero at
 //    rest), u64 epoch flags, the split-K fixup counters and the u64 epoch flags that groups of XCDs read
 //    from one another. Every kernel keeps its data at kWsDataBase and above.
 //  * Epoch flags derive from the launch sequence (epoch = seq << 32 + n), so a flag left by any
@@ -59,7 +59,7 @@ constexpr uint32_t kWsMaxCounters = 1024;
 constexpr uint32_t kWsGroupFlags = 16384;  // [8 XCD][32 rank][4 wave] u64
 constexpr uint32_t kWsDataBase = 24576;
 constexpr unsigned kOwnerPi05Bs1 = 1, kOwnerPi05Batched = 2, kOwnerMa2Bs1 = 3, kOwnerMa2Generic = 4,
-                   kOwnerPrefill = 5, kOwnerPi05Group = 6, kOwnerMa2Group = 7;
+                   kOwnerPrefill = 5, kOwnerPi05Group = 6, kOwnerMa2Group = 7, kOwnerMa2Bs1Long = 8;
 
 __device__ __forceinline__ rsrc_t make_rsrc(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, kRsrcWord3);

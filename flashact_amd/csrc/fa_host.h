@@ -60,7 +60,7 @@ int pi05_bs1_coop_capacity(int device);
 
 // Batch-1 MolmoAct2 launch (XCD-local layout), dispatched from fa_ma2_flow when eligible.
 bool ma2_bs1_eligible(int batch, int Tv, int Lkmax);
-size_t ma2_bs1_workspace_bytes();
+size_t ma2_bs1_workspace_bytes(int Lkmax);
 int ma2_bs1_launch(const fa_ma2_args* a, fa_stream_t stream);
 
 // MolmoAct2 batches of up to 16 samples on groups of XCDs (ma2_group.hip).

@@ -768,7 +768,7 @@ using namespace fa;
 
 extern "C" size_t fa_ma2_workspace_bytes(int batch, int Tv, int Lkmax) {
   if (batch < 1 || Tv < 1 || Tv > ma2::MAX_TV || Lkmax < 16 || (size_t)batch * Tv > (size_t)ma2::MAX_TOKENS) return 0;
-  if (ma2_bs1_eligible(batch, Tv, Lkmax)) return ma2_bs1_workspace_bytes();
+  if (ma2_bs1_eligible(batch, Tv, Lkmax)) return ma2_bs1_workspace_bytes(Lkmax);
   const size_t n = ma2::layout_for(batch, Tv, Lkmax).total;
   if (n >= 0xffffffffull) return 0;
   return ma2_group_eligible(batch, Tv) ? std::max(n, ma2_group_workspace_bytes(batch, Tv)) : n;

@@ -61,6 +61,9 @@ constexpr uint32_t X_H = X_CML + NR * TP * 8;         // [32][384] bf16 fragment
 constexpr uint32_t XB = (X_H + TP * 384 * 2 + 4095) / 4096 * 4096;
 constexpr uint32_t OFF_XCD = OFF_XP + XP_BYTES;
 constexpr uint32_t WS_BYTES = OFF_XCD + NX * XB;
+// Exchange of the kernel for contexts past 512 keys, in whole fp32 values: [4 buffers][8 XCD][32 tokens][768]
+constexpr uint32_t OFF_XW = WS_BYTES, XW_BYTES = 2 * XP_BYTES;
+constexpr uint32_t WS_BYTES_LONG = OFF_XW + XW_BYTES;
 static_assert(OFF_XFLAG + NX * NR * 4 * 8 <= kWsCounters, "flags stay below the fixup counters");
 
 // ---- LDS
@@ -116,6 +119,26 @@ __device__ __forceinline__ u32x4 tag(f32x4 v, unsigned par) {
 __device__ __forceinline__ unsigned mism(u32x4 v, unsigned par) {
   return ((v[0] ^ par) | (v[1] ^ par) | (v[2] ^ par) | (v[3] ^ par)) & 1u;
 }
+// Contexts past 512 keys (WHOLE) exchange all 32 bits of a partial sum. A slot that holds no value yet is
+// all ones, a NaN that the producers never store, and the values themselves say that they have arrived.
+// Four buffers: behind its values of exchange e a wave sets its slots of e + 2 back to all ones. By then
+// every XCD has read e - 2, which lay there: this XCD has read e - 1, whose producers had all read e - 2.
+// The drain of the barrier after the norm puts the reset before the wave's values of e + 1, and whoever
+// polls for e + 2 has read those. A chunk at Lk = 777 takes 9.98 ms, with tagged values 9.70; the displaced
+// bits in a word of their own beside each 16 bytes 10.22, three buffers reset one barrier ahead 10.62.
+__device__ __forceinline__ u32x4 whole(f32x4 v) {
+  u32x4 u = as_u32x4(v);
+#pragma unroll
+  for (int i = 0; i < 4; i++) u[i] = min(u[i], 0xfffffffeu);
+  return u;
+}
+__device__ __forceinline__ bool absent(u32x4 v) { return max(max(v[0], v[1]), max(v[2], v[3])) == 0xffffffffu; }
+template <bool WHOLE>
+constexpr uint32_t kOffX = WHOLE ? OFF_XW : OFF_XP;
+template <bool WHOLE>
+__device__ __forceinline__ unsigned stale(u32x4 v, unsigned par) {
+  return WHOLE ? (unsigned)absent(v) : mism(v, par);
+}
 __device__ __forceinline__ bool aborted(const Ctx& c) {
   return __hip_atomic_load(c.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kErrSpin;
 }
@@ -164,14 +187,15 @@ __device__ __forceinline__ void xwait(Ctx& c) {
 // Wave w reads XCDs 2w, 2w+1 (columns 4 lane + 256 k, k < 3): polls a hint word per XCD with a
 // sleep, loads everything, re-reads groups whose parity is stale; the pair sum goes to LDS and
 // wave 0 adds the 4 pair sums in a fixed order (every XCD computes the same x).
+template <bool WHOLE>
 __device__ __forceinline__ void xread_token(const Ctx& c, int buf, int t, unsigned par, f32x4 (&sum)[3]) {
-  const uint32_t b0 = OFF_XP + (uint32_t)((((buf * NX + 2 * c.w) * TP + t) * D + 4 * c.lane) * 4);
+  const uint32_t b0 = kOffX<WHOLE> + (uint32_t)((((buf * NX + 2 * c.w) * TP + t) * D + 4 * c.lane) * 4);
   const uint32_t xs = (uint32_t)(TP * D * 4);  // next XCD
   if (!aborted(c)) {
-    const uint32_t hint = OFF_XP + (uint32_t)((((buf * NX + 2 * c.w + (c.lane & 1)) * TP + t) * D + D - 4) * 4);
+    const uint32_t hint = kOffX<WHOLE> + (uint32_t)((((buf * NX + 2 * c.w + (c.lane & 1)) * TP + t) * D + D - 4) * 4);
     for (unsigned it = 0;; ++it) {
       const u32x4 h = ldb128<kCpSc1>(c.ws, hint);
-      if (__builtin_amdgcn_ballot_w64(c.lane < 2 && mism(h, par)) == 0) break;
+      if (__builtin_amdgcn_ballot_w64(c.lane < 2 && stale<WHOLE>(h, par)) == 0) break;
       if ((it & 1023) == 1023 && (aborted(c) || it > kSpinCap)) break;
       __builtin_amdgcn_s_sleep(4);
     }
@@ -186,7 +210,7 @@ __device__ __forceinline__ void xread_token(const Ctx& c, int buf, int t, unsign
 #pragma unroll
     for (int x = 0; x < 2; x++)
 #pragma unroll
-      for (int k = 0; k < 3; k++) bad |= mism(v[x][k], par) << (x * 3 + k);
+      for (int k = 0; k < 3; k++) bad |= stale<WHOLE>(v[x][k], par) << (x * 3 + k);
     if (__builtin_amdgcn_ballot_w64(bad != 0) == 0) break;
     if ((it & 255) == 255 && (aborted(c) || it > kSpinCap)) {
       if (c.lane == 0) atomicOr(c.err, kErrSpin);
@@ -216,13 +240,13 @@ __device__ __forceinline__ void xread_token(const Ctx& c, int buf, int t, unsign
 // ---- norm stages (token t = rank r, wave 0 after the exchange read) ---------------------------
 // MODE 0: x = embed(x_t); MODE 1: x += gate * (sum + bias); MODE 2: as 1, then the final norm,
 // the action projection and x_t[:, :adim] += dt * v.
-template <int MODE>
+template <int MODE, bool WHOLE>
 __device__ __forceinline__ void stage_norm(const Params& p, const Ctx& c, int buf, unsigned par, const float* bias,
                                            const float* gate, const float* scale, const float* shift, float dt) {
   const int t = c.r;
   if (t >= p.Tv) return;
   f32x4 sum[3];
-  if (MODE != 0) xread_token(c, buf, t, par, sum);
+  if (MODE != 0) xread_token<WHOLE>(c, buf, t, par, sum);
   if (c.w != 0) return;
   float* xres = reinterpret_cast<float*>(lds + L_X);
   float* xt = reinterpret_cast<float*>(lds + L_XT);
@@ -336,8 +360,8 @@ __device__ __forceinline__ int row24(int base, int rt, int lr) { return base + 1
 
 // Partial-sum projection of this XCD's K-window onto 24 output rows (SO / CO: K = 96 over the
 // head's attention output; DN: K = 384 over h). Wave w = (row tile w / 2, token tile w % 2); the
-// tagged fp32 partial goes to exchange buffer `buf` with the parity bit `par`.
-template <int NK, class WF>
+// fp32 partial goes to exchange buffer `buf`, tagged with the parity bit `par` or whole.
+template <int NK, bool WHOLE, class WF>
 __device__ __forceinline__ void proj24(const Params& p, const Ctx& c, const WF& wf, uint32_t act, int KS,
                                        int buf, unsigned par) {
   const int rt = c.w >> 1, tt = c.w & 1;
@@ -353,9 +377,9 @@ __device__ __forceinline__ void proj24(const Params& p, const Ctx& c, const WF& 
   if (rt == 0 || c.lq < 2) {
     const int col = 24 * c.r + 16 * rt + 4 * c.lq;
     if (t >= p.Tv) acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    __builtin_amdgcn_raw_buffer_store_b128(tag(acc, par), c.ws,
-                                           OFF_XP + (uint32_t)((((buf * NX + c.g) * TP + t) * D + col) * 4), 0,
-                                           kCpSc1);
+    const uint32_t o = (uint32_t)(((c.g * TP + t) * D + col) * 4), xb = (uint32_t)(NX * TP * D * 4);
+    stb128<kCpSc1>(c.ws, kOffX<WHOLE> + buf * xb + o, WHOLE ? whole(acc) : tag(acc, par));
+    if (WHOLE) stb128<kCpSc1>(c.ws, kOffX<WHOLE> + (buf ^ 2) * xb + o, u32x4{~0u, ~0u, ~0u, ~0u});
   }
 }
 
@@ -646,10 +670,12 @@ __device__ __forceinline__ void mark(const Params& p, int idx, uint64_t& t0) {
   }
 }
 
-// NC: context chunk slots of the combine, 16 (Lk <= 512: 9.59 ms per chunk at Lk = 493) or 32 (9.71 ms
-// at Lk = 777, which took 27.6 ms on the stage-engine kernel).
+// NC: context chunk slots of the combine, 16 (Lk <= 512: 9.59 ms per chunk at Lk = 493) or 32 (9.98 ms
+// at Lk = 777, which took 27.6 ms on the stage-engine kernel, whose partial sums are whole fp32 too).
 template <int NC>
 __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
+  constexpr bool WHOLE = NC > NR / 2;
+  constexpr unsigned OWNER = WHOLE ? kOwnerMa2Bs1Long : kOwnerMa2Bs1;  // the state below differs
   Ctx c;
   c.g = blockIdx.x & 7;
   c.r = blockIdx.x >> 3;
@@ -669,13 +695,14 @@ __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
   const unsigned owner =
       __hip_atomic_load(reinterpret_cast<const unsigned*>(p.ws + kWsOwner), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (threadIdx.x == 0 && xcc_id() != (unsigned)c.g) atomicOr(c.err, kErrXcd);
-  if (owner != kOwnerMa2Bs1) {
+  if (owner != OWNER) {
     // Another kernel used the workspace since this one last did: its data may sit in the exchange
-    // buffers with any parity. Clear them (parity 0), restart the parity sequence and pass one
-    // grid barrier before the first exchange.
+    // buffers with any parity. Clear them (parity 0, or no value), restart the parity (buffer) sequence
+    // and pass one grid barrier before the first exchange.
     base0 = base1 = 0;
-    for (uint32_t i = blockIdx.x * NTHR + threadIdx.x; i < XP_BYTES / 16; i += NWG * NTHR)
-      stb128<kCpSc1>(c.ws, OFF_XP + 16 * i, u32x4{0u, 0u, 0u, 0u});
+    constexpr unsigned fill = WHOLE ? ~0u : 0u;
+    for (uint32_t i = blockIdx.x * NTHR + threadIdx.x; i < (WHOLE ? XW_BYTES : XP_BYTES) / 16; i += NWG * NTHR)
+      stb128<kCpSc1>(c.ws, kOffX<WHOLE> + 16 * i, u32x4{fill, fill, fill, fill});
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     c.e += 1;
@@ -694,7 +721,8 @@ __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
   }
   __syncthreads();
   // exchange e uses buffer e & 1; the n-th use of a buffer carries parity (1 + base + n) & 1
-  auto buf = [](int e) { return e & 1; };
+  // (WHOLE: buffer (base + e) & 3)
+  auto buf = [&](int e) { return WHOLE ? (int)((base0 + (unsigned)e) & 3u) : e & 1; };
   auto par = [&](int e) { return (1u + ((e & 1) ? base1 : base0) + (unsigned)(e >> 1)) & 1u; };
   const int NL = p.NL;
   auto copy_qkv = [&](int l) {  // waves 2 and 3: the QKV weights of ranks 0..17
@@ -714,9 +742,9 @@ __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
       const int e0 = 3 * li, e1 = e0 + 1, e2 = e0 + 2;
       // N_msa
       if (l == 0)
-        stage_norm<0>(p, c, 0, 0u, nullptr, nullptr, mo, mo + D, 0.f);
+        stage_norm<0, WHOLE>(p, c, 0, 0u, nullptr, nullptr, mo, mo + D, 0.f);
       else
-        stage_norm<1>(p, c, buf(e0 - 1), par(e0 - 1), p.b_dn + (size_t)(l - 1) * D, mo - 9 * D + 8 * D, mo, mo + D,
+        stage_norm<1, WHOLE>(p, c, buf(e0 - 1), par(e0 - 1), p.b_dn + (size_t)(l - 1) * D, mo - 9 * D + 8 * D, mo, mo + D,
                       0.f);
       mark(p, 0, t0);
       xarrive(c);
@@ -751,7 +779,7 @@ __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
       xwait(c);
       mark(p, 15, t0);
       // SO -> exchange e0
-      proj24<3>(p, c, [&](int j) { return wso[j]; }, X_ATT, 3, buf(e0), par(e0));
+      proj24<3, WHOLE>(p, c, [&](int j) { return wso[j]; }, X_ATT, 3, buf(e0), par(e0));
       mark(p, 3, t0);
       // N_mca, with this rank's context keys/values in flight
       u32x4 kf[2][3], vf[6];
@@ -771,7 +799,7 @@ __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
         for (int dt2 = 0; dt2 < 6; dt2++)
           vf[dt2] = *reinterpret_cast<const u32x4*>(V + (size_t)(HD * c.g + 16 * dt2 + c.lr) * p.Lkmax + kg);
       }
-      stage_norm<1>(p, c, buf(e0), par(e0), p.b_so + (size_t)l * D, mo + 2 * D, mo + 3 * D, mo + 4 * D, 0.f);
+      stage_norm<1, WHOLE>(p, c, buf(e0), par(e0), p.b_so + (size_t)l * D, mo + 2 * D, mo + 3 * D, mo + 4 * D, 0.f);
       mark(p, 4, t0);
       xarrive(c);
       xwait(c);
@@ -812,10 +840,10 @@ __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
       xwait(c);
       mark(p, 15, t0);
       // CO -> exchange e1
-      proj24<3>(p, c, [&](int j) { return wco[j]; }, X_ATT, 3, buf(e1), par(e1));
+      proj24<3, WHOLE>(p, c, [&](int j) { return wco[j]; }, X_ATT, 3, buf(e1), par(e1));
       mark(p, 8, t0);
       // N_mlp
-      stage_norm<1>(p, c, buf(e1), par(e1), p.b_co + (size_t)l * D, mo + 5 * D, mo + 6 * D, mo + 7 * D, 0.f);
+      stage_norm<1, WHOLE>(p, c, buf(e1), par(e1), p.b_co + (size_t)l * D, mo + 5 * D, mo + 6 * D, mo + 7 * D, 0.f);
       mark(p, 9, t0);
       xarrive(c);
       xwait(c);
@@ -827,23 +855,22 @@ __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
       xwait(c);
       mark(p, 15, t0);
       // DN -> exchange e2
-      proj24<12>(p, c, [&](int j) { return lds128(L_DN + ((c.w >> 1) * 12 + j) * 1024 + frag_slot(c.lr, c.lq)); }, X_H, 12, buf(e2), par(e2));
+      proj24<12, WHOLE>(p, c, [&](int j) { return lds128(L_DN + ((c.w >> 1) * 12 + j) * 1024 + frag_slot(c.lr, c.lq)); }, X_H, 12, buf(e2), par(e2));
       mark(p, 11, t0);
     }
     const int el = 3 * (step * NL + NL - 1) + 2;
     const float* ml = p.mods + ((size_t)step * NL + NL - 1) * 9 * D;
     const float* mf = p.mod_final + (size_t)step * 2 * D;
-    stage_norm<2>(p, c, buf(el), par(el), p.b_dn + (size_t)(NL - 1) * D, ml + 8 * D, mf, mf + D, dt);
+    stage_norm<2, WHOLE>(p, c, buf(el), par(el), p.b_dn + (size_t)(NL - 1) * D, ml + 8 * D, mf, mf + D, dt);
     mark(p, 12, t0);
   }
   if (c.g == 0 && c.w == 0 && c.lane < AD && c.r < p.Tv) p.x_t[c.r * AD + c.lane] = xt[c.lane];
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     const unsigned n = 3u * (unsigned)(p.S * NL);  // exchanges in this launch
     unsigned* pw = reinterpret_cast<unsigned*>(p.ws + OFF_CTRL + 12);
-    __hip_atomic_store(pw, (base0 + (n + 1) / 2) & 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(pw + 1, (base1 + n / 2) & 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(reinterpret_cast<unsigned*>(p.ws + kWsOwner), kOwnerMa2Bs1, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(pw, WHOLE ? (base0 + n) & 3u : (base0 + (n + 1) / 2) & 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(pw + 1, WHOLE ? 0u : (base1 + n / 2) & 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(reinterpret_cast<unsigned*>(p.ws + kWsOwner), OWNER, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(reinterpret_cast<uint64_t*>(p.ws + OFF_CTRL), seq + 1, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
   }
@@ -855,13 +882,15 @@ __global__ void __launch_bounds__(NTHR, 1) ma2x_kernel(Params p) {
 bool ma2_bs1_eligible(int batch, int Tv, int Lkmax) {
   return batch == 1 && Tv <= ma2x::TP && Lkmax <= ma2x::MAX_LK;
 }
-size_t ma2_bs1_workspace_bytes() { return ma2x::WS_BYTES; }
+size_t ma2_bs1_workspace_bytes(int Lkmax) {
+  return Lkmax <= ma2x::NR / 2 * ma2x::KPR ? ma2x::WS_BYTES : ma2x::WS_BYTES_LONG;
+}
 
 int ma2_bs1_launch(const fa_ma2_args* a, fa_stream_t stream) {
   using namespace fa::ma2x;
-  if (a->workspace_bytes < WS_BYTES)
-    return host::fail(FA_ERR_INVALID_ARG, "fa_ma2_flow: workspace_bytes=%zu < required %u", a->workspace_bytes,
-                      (unsigned)WS_BYTES);
+  const size_t need = ma2_bs1_workspace_bytes(a->Lkmax);
+  if (a->workspace_bytes < need)
+    return host::fail(FA_ERR_INVALID_ARG, "fa_ma2_flow: workspace_bytes=%zu < required %zu", a->workspace_bytes, need);
   // Up to 512 keys the combine's sixteen chunk slots are enough (half the loads); past that, 32.
   const void* kern = a->Lk <= NR / 2 * KPR ? (const void*)ma2x_kernel<NR / 2> : (const void*)ma2x_kernel<NR>;
   int rc = host::check_device(kern, NTHR, LDS_BYTES, NWG, "fa_ma2_flow");

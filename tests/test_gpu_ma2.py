@@ -57,6 +57,26 @@ def test_ma2_long_context(gpu, Lk, Tv):
     _check(C.make_case(NL=2, Lk=Lk, Tv=Tv, S=2, seed=Lk), gpu)
 
 
+def test_ma2_long_context_keeps_whole_partial_sums(gpu):
+    """Past 512 keys the batch-1 kernel's exchanged partial sums are whole fp32 values: launches whose
+    exchanges carry other parities (one layer and one step make three, so the parity of the second
+    exchange buffer flips from launch to launch) give the same bits, also after the kernel of the shorter
+    contexts has used the workspace."""
+    import torch
+    c = C.make_case(NL=1, Lk=600, Tv=32, S=1, adim=32, seed=3)
+    short = C.make_case(NL=1, Lk=90, Tv=32, S=1, adim=32, seed=4)
+    n = ma2.workspace(gpu, 1, 32, ma2.lkmax_for(600)).numel()
+    raw = torch.zeros(n + 256, dtype=torch.uint8, device=gpu)
+    ws = raw[(-raw.data_ptr()) % 256:][:n]
+    first = C.run_gpu(c, gpu, ws=ws)
+    for again in range(3):
+        assert np.array_equal(C.run_gpu(c, gpu, ws=ws), first), again
+    C.run_gpu(short, gpu, ws=ws)
+    assert np.array_equal(C.run_gpu(c, gpu, ws=ws), first)
+    assert np.array_equal(C.run_gpu(c, gpu, ws=ws), first)
+    assert ma2.read_status(ws) == 0
+
+
 # Batch 1, layer counts whose next layer is the same (1) and an odd one, a single token, a full second token
 # tile and the last row of the first, contexts that leave ranks without keys: the layer's weights lie in LDS
 # regions that other stages and the next layer reuse. Four steps, as for the groups below.
