@@ -550,6 +550,12 @@ __device__ __forceinline__ void stage_catt(const Params& p, const MCtx& c, int p
   for (int dt = 0; dt < 6; dt++) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
   for (int b0 = 0; b0 < c.nblk; b0 += SB) {
+    // TT = 2: the last segment may hold no block of this wave; m, l and O then stay. (A softmax over masked
+    // scores alone would weigh them exp2(rounding error of -1e30 qscale): 0 here, infinite for some scales.)
+    if (b0 + pr >= c.nblk) {
+      page_release<K>(c, pgk + c.nblk);
+      break;
+    }
     f32x4 s[2 * NBK];
 #pragma unroll
     for (int i = 0; i < NBK; i++) {

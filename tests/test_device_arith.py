@@ -8,6 +8,11 @@ neighbours one ulp away, which brackets v_rcp_f32's result, and the quotient and
 compared with numpy's integer division over every m below 2^18 for the divisors the kernels see
 (every d up to 256, the pi0.5 and MolmoAct2 token counts and their multiples by the head count) and
 a spread of others up to 2^18. A planted mistake (the correction step left out) must fail.
+
+Also the softmax over key segments of the attention that shares a token tile among two waves
+(stage_catt of ma2_group.hip), restated for one query row: the fold exp2(fma(s, qscale, -m)) weighs
+masked scores by the rounding error of -1e30 qscale, so a wave must leave out a segment in which no
+block is its own.
 """
 import numpy as np
 
@@ -49,3 +54,44 @@ def test_divmod_u_needs_its_correction_step():
             q, _ = _divmod_float(m, d, rd, correct=False)
             wrong += int((q != m // d).sum())
     assert wrong > 0
+
+
+MASKED = np.float32(-1e30)
+
+
+def _softmax_state(segments, qscale, skip=True):
+    """(m, l) of one wave and query row after segments of raw scores; None: no block of it is the wave's."""
+    m, l = MASKED, np.float32(0)
+    for seg in segments:
+        if seg is None and skip:
+            continue
+        x = np.full(64, MASKED) if seg is None else np.asarray(seg, np.float32)
+        new = max(m, np.float32(x.max() * qscale))
+        with np.errstate(over="ignore", under="ignore"):
+            alpha = np.exp2(np.float64(m) - np.float64(new)).astype(np.float32)
+            # fma: the product of two float32 is exact in float64
+            w = np.exp2((x.astype(np.float64) * np.float64(qscale) - np.float64(new)).astype(np.float32))
+            l = np.float32(l * alpha + w.sum(dtype=np.float32))
+        m = new
+    return m, l
+
+
+def _qscale(head_dim):  # as the kernels round it: log2(e) times 1 / sqrt(head_dim), both float32
+    return np.float32(1.4426950408889634) * np.float32(1.0 / np.sqrt(head_dim))
+
+
+def test_segment_without_a_block_has_no_weight():
+    rng = np.random.default_rng(0)
+    for hd in (64, 80, 96, 128, 192, 256):
+        q, keys = _qscale(hd), rng.standard_normal(64).astype(np.float32) * 8
+        m, l = _softmax_state([None], q)
+        assert l == 0 and np.isfinite(m)
+        alone, led = _softmax_state([keys], q), _softmax_state([None, keys], q)
+        assert alone == led == _softmax_state([keys, None], q), hd
+        ref = np.exp2(keys.astype(np.float64) * np.float64(q))
+        assert abs(np.float64(alone[1]) * np.exp2(np.float64(alone[0])) / ref.sum() - 1) < 1e-5
+
+
+def test_segment_without_a_block_needs_its_skip():
+    states = [_softmax_state([None], _qscale(hd), skip=False)[1] for hd in (64, 80, 96, 128, 192, 256)]
+    assert np.isinf(states).any()
