@@ -43,6 +43,7 @@ int pi05_check_batched(const fa_pi05_args* a);
 // Batches of 2 to 16 samples on groups of XCDs (pi05_group.hip).
 bool pi05_group_eligible(int batch, int Tv);
 size_t pi05_group_workspace_bytes(int batch);
+bool pi05_group_faster(int batch, int Tv, int Lp);  // than the stage engine
 int pi05_denoise_group(const fa_pi05_args* a, fa_stream_t stream);
 
 // K/V hand-off (srows > 0): enqueues the de-interleave / transpose of kvsrc_k / kvsrc_v into the

@@ -1,7 +1,7 @@
-// pi0.5 action-expert denoise loop for batches past 16 samples, and for smaller ones whose workspace has
-// no room for the group kernel (pi05_group.hip): the whole S-step Euler loop in ONE cooperative launch of 256
-// workgroups x 4 waves, built on the stage engine (engine.h). This is the MFMA-bound regime, so
-// the GEMMs are 128-token tiles over all samples at once.
+// pi0.5 action-expert denoise loop for batches past 16 samples, and for smaller ones with long prefixes
+// or whose workspace has no room for the group kernel (pi05_group.hip): the whole S-step Euler loop in ONE
+// cooperative launch of 256 workgroups x 4 waves, built on the stage engine (engine.h). This is the
+// MFMA-bound regime, so the GEMMs are 128-token tiles over all samples at once.
 //
 // Per layer (grid barrier after each stage), token m = b * Tv + t of sample b:
 //   N1   x = embed(x_t) (layer 0) or x += gate_post * sum(down partials); xn = adaRMS(x)

@@ -1460,9 +1460,10 @@ extern "C" int fa_pi05_denoise(const fa_pi05_args* a, fa_stream_t stream) {
   if (a->batch > 1) {
     const int rc = pi05_check_batched(a);
     if (rc != FA_OK) return rc;
-    // Up to 16 samples, groups of XCDs; past that (or in a workspace too small for the groups) the
-    // stage engine, whose GEMM tiles are then full.
-    if (pi05_group_eligible(a->batch, a->Tv) && a->workspace_bytes >= pi05_group_workspace_bytes(a->batch))
+    // Up to 16 samples, groups of XCDs; past that, whose tokens fill the stage engine's GEMM tiles, for long
+    // prefixes of 9 and more samples, and in a workspace too small for the groups, the stage engine.
+    if (pi05_group_eligible(a->batch, a->Tv) && pi05_group_faster(a->batch, a->Tv, a->Lp) &&
+        a->workspace_bytes >= pi05_group_workspace_bytes(a->batch))
       return pi05_denoise_group(a, stream);
     return pi05_denoise_batched(a, stream);
   }

@@ -51,6 +51,24 @@ def test_batched_group_shapes(gpu, B, Lp, Tv, S, NL):
     _check(P.make_case(NL=NL, Lp=Lp, Tv=Tv, S=S, batch=B, seed=B + Lp + Tv), gpu)
 
 
+OWNER_STAGE, OWNER_GROUP = 2, 6  # the workspace's owner word (u32 at byte 20): the kernel that ran last
+
+
+def _owner(ws):
+    return int(ws[20:24].view(torch.int32).item())
+
+
+# Long prefixes of 9 to 16 samples run on whichever kernel is faster there, short horizons on the stage
+# engine: each side of the rule, and the shortest prefix past it at 9 samples (2689) and its neighbour.
+@pytest.mark.parametrize("B,Lp,Tv,owner", [(9, 2688, 10, OWNER_GROUP), (9, 2689, 10, OWNER_STAGE), (16, 8100, 1, OWNER_STAGE),
+                                          (12, 4200, 33, OWNER_GROUP), (12, 8128, 64, OWNER_GROUP), (8, 8100, 1, OWNER_GROUP)])
+def test_batched_long_prefixes(gpu, B, Lp, Tv, owner):
+    c = P.make_case(NL=1, Lp=Lp, Tv=Tv, S=1, batch=B, seed=B + Tv)
+    _check(c, gpu)
+    ws = pi05.workspace(gpu, B, Tv, pi05.lmax_for(Lp, Tv))
+    assert _owner(ws) == owner
+
+
 def test_batched_repeats_on_one_workspace(gpu):
     """Launches of different group shapes, of the batch-1 kernel and of the stage engine (a workspace too
     small for the groups) on one workspace, each against its first result."""
