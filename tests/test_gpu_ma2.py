@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from tests import ma2_case as C
+from tests import stage_engine as SE
 from flashact_amd import ma2
 
 MAX_ABS, MEAN_ABS = 2e-2, 2e-3
@@ -39,8 +40,8 @@ def test_ma2_config4_bs1(gpu):
 
 
 # Batch 1 runs the XCD-local kernel up to Tv = 32 and Lk = 1024: (1, 512, 32) fills every token lane
-# and context rank; (1, 65, 17) leaves one token in the second token tile and a ragged key chunk.
-# (1, 300, 40) runs the generic kernel's small-tile path with four waves per cross-attention item.
+# and context rank; (1, 65, 17) leaves one token in the second token tile and a ragged key chunk. The
+# others run the group kernels (one sample with 40 tokens too).
 @pytest.mark.parametrize("B,Lk,Tv,S,adim", [(1, 1, 1, 2, 6), (2, 700, 64, 1, 32), (3, 37, 17, 2, 5),
                                             (1, 128, 16, 1, 6), (2, 129, 33, 1, 1), (1, 512, 32, 2, 6),
                                             (1, 65, 17, 2, 7), (1, 300, 40, 2, 6)])
@@ -49,9 +50,9 @@ def test_ma2_edge_shapes(gpu, B, Lk, Tv, S, adim):
 
 
 # Contexts past 512 rows at batch 1: one key in the 17th chunk (513), a ragged chunk (777), every rank
-# attending (1024) and the first context of the stage-engine kernel. Two steps: one Euler step of
-# dt = 1 with unit gates sits at 2e-3 mean-abs from its bf16 operands alone (the stage-engine kernel
-# 2.3e-3 at Lk = 1025, Tv = 5), two at 1.5e-3.
+# attending (1024) and the first context of the group kernel. Two steps: one Euler step of dt = 1 with
+# unit gates sits at 2e-3 mean-abs from its bf16 operands alone (the stage-engine kernel 2.3e-3 at
+# Lk = 1025, Tv = 5), two at 1.5e-3.
 @pytest.mark.parametrize("Lk,Tv", [(513, 30), (777, 17), (1024, 32), (1025, 5)])
 def test_ma2_long_context(gpu, Lk, Tv):
     _check(C.make_case(NL=2, Lk=Lk, Tv=Tv, S=2, seed=Lk), gpu)
@@ -97,6 +98,42 @@ def test_ma2_group_shapes(gpu, B, Lk, Tv, adim):
     _check(C.make_case(NL=2, Lk=Lk, Tv=Tv, S=4, adim=adim, batch=B, seed=B + Lk + Tv), gpu)
 
 
+def _check_stage(c, gpu, ws=None):
+    ref = C.run_oracle(c)
+    ws = ws if ws is not None else ma2.workspace(gpu, c["batch"], c["Tv"], ma2.lkmax_for(c["Lk"]))
+    out = C.run_gpu(c, gpu, ws=ws)
+    assert ma2.read_status(ws) == 0 and SE.owner(ws) == SE.MA2_STAGE
+    for b in range(c["batch"]):
+        st = C.parity(out[b, :c["Tv"]], ref[b], c["adim"])
+        print(f"stage B={c['batch']} sample {b} NL={c['NL']} Lk={c['Lk']} Tv={c['Tv']} S={c['S']}: {st}", flush=True)
+        assert st["max_abs"] <= MAX_ABS and st["mean_abs"] <= MEAN_ABS, (b, st)
+        assert np.all(out[b, :c["Tv"], c["adim"]:] == c["inp"]["noise"][b, :, c["adim"]:].numpy())
+    return out
+
+
+# The stage engine where it serves, past 16 samples: its small tiles (up to 64 tokens, split-K sums in place)
+# and its large ones, partial and full, up to 2048 tokens. Four steps, as for the groups.
+@pytest.mark.parametrize("B,Lk,Tv,adim,NL", [(17, 300, 3, 32, 3), (64, 33, 1, 32, 2), (17, 493, 30, 6, 2), (20, 1100, 33, 6, 2),
+                                            (32, 129, 64, 32, 2)])
+def test_ma2_stage_engine_large_batches(gpu, B, Lk, Tv, adim, NL):
+    _check_stage(C.make_case(NL=NL, Lk=Lk, Tv=Tv, S=4, adim=adim, batch=B, seed=B + Lk + Tv), gpu)
+
+
+def test_ma2_stage_engine_full_depth(gpu):
+    _check_stage(C.make_case(NL=36, Lk=493, Tv=30, S=10, batch=17, seed=6), gpu)
+
+
+# Batches that fit the groups, on a workspace without room for them (the stage engine needs less up to 64
+# tokens): its small tiles with one to four waves per cross-attention item. Run twice: the split-K counters
+# are back at zero.
+@pytest.mark.parametrize("B,Lk,Tv,adim", [(1, 300, 40, 6), (1, 1025, 5, 32), (2, 129, 30, 6), (3, 37, 17, 5), (1, 128, 64, 32)])
+def test_ma2_stage_engine_small_batches(gpu, B, Lk, Tv, adim):
+    c = C.make_case(NL=2, Lk=Lk, Tv=Tv, S=4, adim=adim, batch=B, seed=B + Lk + Tv)
+    ws = SE.zeroed(SE.need(lambda w: C.run_gpu(c, gpu, ws=w), gpu), gpu)
+    first = _check_stage(c, gpu, ws)
+    assert np.array_equal(C.run_gpu(c, gpu, ws=ws), first)
+
+
 def test_ma2_groups_repeat_on_one_workspace(gpu):
     """Launches of different group shapes and of the stage engine (a workspace with no room for the groups)
     on one workspace, each against its first result."""
@@ -116,7 +153,7 @@ def test_ma2_groups_repeat_on_one_workspace(gpu):
 
 
 def test_ma2_batch16(gpu):
-    """The MolmoAct2 benchmark workload at batch 16 (the large-tile path) at full depth, 36 layers x 10 steps, every
+    """The MolmoAct2 benchmark workload at batch 16 (on the groups) at full depth, 36 layers x 10 steps, every
     sample against the oracle (benchmarks/molmoact2/eval_numerics.py:147-159 is the reference's
     fidelity check of the same loop)."""
     _check(C.make_case(NL=36, Lk=493, Tv=30, S=10, batch=16), gpu)

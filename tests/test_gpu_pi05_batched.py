@@ -1,4 +1,5 @@
-"""Batched pi0.5 denoise loop (batch >= 2: the MFMA-bound kernel) on the MI355X vs the CPU fp32 oracle.
+"""Batched pi0.5 denoise loop (batch >= 2) on the MI355X vs the CPU fp32 oracle: the group kernels (2 to 16
+samples) and the stage engine (more, long prefixes, workspaces without room for the groups).
 
 Tolerance (the acceptance tolerance for bf16 operands with fp32 accumulation vs the fp32 oracle, on the
 final actions of every sample): max-abs <= 2e-2 and mean-abs <= 2e-3.
@@ -8,6 +9,7 @@ import pytest
 import torch
 
 from tests import pi05_case as P
+from tests import stage_engine as SE
 from flashact_amd import pi05
 
 MAX_ABS, MEAN_ABS = 2e-2, 2e-3
@@ -32,8 +34,9 @@ def test_batched_two_samples(gpu):
     _check(P.make_case(NL=2, Lp=968, Tv=50, S=2, batch=2), gpu)
 
 
-# Lp + Tv: 54, 50, 364, 1109 end inside a 128-key chunk (the last chunk masked, its V^T tail group
-# zeroed), 256 fills every chunk exactly (no masking at all)
+# Lp + Tv: 54, 50, 364, 1109 end inside a 128-key chunk of the stage engine (the last chunk masked, its V^T
+# tail group zeroed), 256 fills every chunk exactly (no masking at all); below on the groups, whose chunks are
+# of the prefix alone, and in test_stage_engine_small_batches on the stage engine
 @pytest.mark.parametrize("B,Lp,Tv,S", [(3, 37, 17, 2), (2, 0, 50, 1), (5, 300, 64, 1), (2, 1100, 9, 2),
                                       (2, 206, 50, 1)])
 def test_batched_edge_shapes(gpu, B, Lp, Tv, S):
@@ -51,22 +54,51 @@ def test_batched_group_shapes(gpu, B, Lp, Tv, S, NL):
     _check(P.make_case(NL=NL, Lp=Lp, Tv=Tv, S=S, batch=B, seed=B + Lp + Tv), gpu)
 
 
-OWNER_STAGE, OWNER_GROUP = 2, 6  # the workspace's owner word (u32 at byte 20): the kernel that ran last
-
-
-def _owner(ws):
-    return int(ws[20:24].view(torch.int32).item())
-
-
 # Long prefixes of 9 to 16 samples run on whichever kernel is faster there, short horizons on the stage
 # engine: each side of the rule, and the shortest prefix past it at 9 samples (2689) and its neighbour.
-@pytest.mark.parametrize("B,Lp,Tv,owner", [(9, 2688, 10, OWNER_GROUP), (9, 2689, 10, OWNER_STAGE), (16, 8100, 1, OWNER_STAGE),
-                                          (12, 4200, 33, OWNER_GROUP), (12, 8128, 64, OWNER_GROUP), (8, 8100, 1, OWNER_GROUP)])
+@pytest.mark.parametrize("B,Lp,Tv,owner", [(9, 2688, 10, SE.PI05_GROUP), (9, 2689, 10, SE.PI05_STAGE),
+                                          (16, 8100, 1, SE.PI05_STAGE), (12, 4200, 33, SE.PI05_GROUP),
+                                          (12, 8128, 64, SE.PI05_GROUP), (8, 8100, 1, SE.PI05_GROUP)])
 def test_batched_long_prefixes(gpu, B, Lp, Tv, owner):
     c = P.make_case(NL=1, Lp=Lp, Tv=Tv, S=1, batch=B, seed=B + Tv)
     _check(c, gpu)
     ws = pi05.workspace(gpu, B, Tv, pi05.lmax_for(Lp, Tv))
-    assert _owner(ws) == owner
+    assert SE.owner(ws) == owner
+
+
+def _check_stage(c, gpu, ws=None):
+    ref = P.run_oracle(c)
+    ws = ws if ws is not None else pi05.workspace(gpu, c["batch"], c["Tv"], pi05.lmax_for(c["Lp"], c["Tv"]))
+    out = P.run_gpu_batched(c, gpu, ws=ws)[0]
+    assert pi05.read_status(ws) == 0 and SE.owner(ws) == SE.PI05_STAGE
+    for b in range(c["batch"]):
+        st = P.parity(out[b, :c["Tv"]], ref[b])
+        print(f"stage B={c['batch']} sample {b} NL={c['NL']} Lp={c['Lp']} Tv={c['Tv']} S={c['S']}: {st}", flush=True)
+        assert st["max_abs"] <= MAX_ABS and st["mean_abs"] <= MEAN_ABS, (b, st)
+    return out
+
+
+# The stage engine where it serves: past 16 samples, several token tiles (the last one partial or full, up to
+# the 4096 tokens of a launch), layers after layers, prefixes of none to more than eight key chunks.
+@pytest.mark.parametrize("B,Lp,Tv,S,NL", [(17, 1100, 50, 2, 3), (18, 0, 64, 2, 2), (40, 206, 50, 2, 2), (64, 70, 64, 2, 2),
+                                         (64, 300, 2, 2, 2)])
+def test_stage_engine_large_batches(gpu, B, Lp, Tv, S, NL):
+    _check_stage(P.make_case(NL=NL, Lp=Lp, Tv=Tv, S=S, batch=B, seed=B + Lp + Tv), gpu)
+
+
+def test_stage_engine_full_depth(gpu):
+    _check_stage(P.make_case(NL=18, Lp=968, Tv=50, S=10, batch=17, seed=5), gpu)
+
+
+# The shapes of test_batched_edge_shapes and the first of this file, and more than 8 samples, on a workspace
+# without room for the groups.
+@pytest.mark.parametrize("B,Lp,Tv,S", [(2, 968, 50, 2), (3, 37, 17, 2), (2, 0, 50, 1), (5, 300, 64, 1), (2, 1100, 9, 2),
+                                      (2, 206, 50, 1), (12, 1100, 17, 2)])
+def test_stage_engine_small_batches(gpu, B, Lp, Tv, S):
+    c = P.make_case(NL=2, Lp=Lp, Tv=Tv, S=S, batch=B, seed=B + Lp + Tv)
+    ws = SE.zeroed(SE.need(lambda w: P.run_gpu_batched(c, gpu, ws=w), gpu), gpu)
+    first = _check_stage(c, gpu, ws)
+    assert np.array_equal(P.run_gpu_batched(c, gpu, ws=ws)[0], first)
 
 
 def test_batched_repeats_on_one_workspace(gpu):
