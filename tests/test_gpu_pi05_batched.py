@@ -161,3 +161,30 @@ def test_batched_suffix_cache_rows(gpu):
         assert torch.allclose(kc[b, 0, 64:72], k, atol=3e-2, rtol=3e-2)
         assert torch.allclose(vc[b, 0, :, 64:72].T, v, atol=3e-2, rtol=3e-2)
         assert torch.equal(kc[b, 0, :64], c["inp"]["kpre"][b, 0].float())
+
+
+# Every group shape with full, partial and absent samples, and the stage engine: the rows of this step's keys
+# and values that a launch leaves in the caches, of every sample and layer, against the batch-1 kernel's.
+# More layers than XCDs of a group, since they take turns writing them; the rows before and behind stay.
+# bf16 rows of layers whose inputs differ by their own bf16 operands: the bound of the test above.
+@pytest.mark.parametrize("B,Lp,Tv", [(2, 70, 33), (3, 64, 64), (4, 37, 17), (5, 129, 50), (8, 70, 9), (9, 65, 16),
+                                    (16, 40, 37), (17, 70, 9)])
+def test_batched_cache_rows_of_every_layer(gpu, B, Lp, Tv):
+    NL = 6
+    c = P.make_case(NL=NL, Lp=Lp, Tv=Tv, S=2, batch=B, seed=B + Lp)
+    g, g1 = P.gpu_tensors(c, gpu), P.gpu_tensors(c, gpu)
+    for k, v in g["caches"]:  # rows that no launch may touch or use
+        k[:, Lp + Tv:], v[..., Lp + Tv:] = 7.0, 7.0
+    _, kc, vc = P.run_gpu_batched(c, gpu, g)
+    ws = pi05.workspace(gpu, B, Tv, g["Lmax"])
+    assert pi05.read_status(ws) == 0
+    assert SE.owner(ws) == (SE.PI05_GROUP if B <= 16 else SE.PI05_STAGE)
+    for b in range(B):
+        _, k1, v1 = P.run_gpu(c, gpu, g1, sample=b)
+        k, v = kc[b].float(), vc[b].float()
+        for l in range(NL):
+            assert torch.allclose(k[l, Lp:Lp + Tv], k1[l, Lp:Lp + Tv].float(), atol=3e-2, rtol=3e-2), (b, l)
+            assert torch.allclose(v[l, :, Lp:Lp + Tv], v1[l, :, Lp:Lp + Tv].float(), atol=3e-2, rtol=3e-2), (b, l)
+        assert torch.equal(k[:, :Lp], c["inp"]["kpre"][b].float().to(gpu))
+        assert torch.equal(v[..., :Lp], c["inp"]["vpre"][b].float().transpose(1, 2).to(gpu))
+        assert (k[:, Lp + Tv:] == 7).all() and (v[..., Lp + Tv:] == 7).all()
