@@ -64,9 +64,9 @@ struct Plan {
            rounds(128 * GW, 2 * FF / 128) * g_us() + rounds(128 * DW, D / DB * KS_DN) * d_us();
   }
 };
-// Prefill of one sample, PlanMax for every size -> the plan taken (ms): Lp 60 2.79 -> 1.87, 129 2.80 -> 2.01,
-// 293 3.04 -> 2.32, 400 3.17 -> 2.66, 561 3.80 -> 3.33, 968 the same plan, 1100 6.16 -> 5.66, 1300 6.92 -> 6.42;
-// four samples of 561: 9.98 -> 9.59. Weights alone take 0.74 ms at 5 TB/s: small counts are bound by the
+// Prefill of one sample, PlanMax for every size -> the plan taken (ms, one run): Lp 60 2.75 -> 1.82, 129 2.76 ->
+// 1.95, 293 2.97 -> 2.27, 450 3.21 -> 2.63, 600 3.71 -> 3.32, 968 the same plan, 1100 6.07 -> 5.55, 1300 6.82 -> 6.34;
+// four samples of 561: 9.75 -> 9.36. Weights alone take 0.74 ms at 5 TB/s: small counts are bound by the
 // chain of seven grid barriers and k-step chains per layer, large ones by the matrix cores.
 using Plan128 = Plan<2, 2, 4, 2, 2, 4, 1, 1, 64>;
 using Plan256 = Plan<2, 2, 4, 2, 2, 4, 2, 2, 64>;

@@ -120,13 +120,16 @@ def test_prefill_batch_matches_single(gpu):
 
 
 def test_prefill_tile_plans(gpu):
-    """Every tile plan and both sides of each of its edges, tokens without neighbours (Lp = 1, so M = batch):
-    the K splits and the k order do not depend on the plan, so a token's K and V are the same bits in all."""
-    M = 1153
+    """Every tile plan and both sides of every token count at which the rule changes plans (the last is 5376),
+    tokens without neighbours (Lp = 1, so M = batch): the K splits and the k order do not depend on the plan, so
+    a token's K and V are the same bits in all."""
+    M = 5378
     c = C.make_case(NL=2, Lp=1, batch=M, seed=12)
     g = C.gpu_weights(c, gpu)
     kr, vr = C.run_gpu(c, gpu, g)
-    for n in (2, 64, 65, 128, 129, 256, 257, 384, 385, 512, 513, 768, 769, 1024, 1025, 1152):
+    for n in (2, 64, 65, 128, 129, 256, 257, 384, 385, 512, 513, 768, 769, 1024, 1025, 1152, 1153, 1536, 1537, 2048,
+              2049, 2304, 2305, 2560, 2561, 2688, 2689, 3584, 3585, 3648, 3649, 3840, 3841, 4096, 4097, 4224, 4225, 5120,
+              5121, 5376, 5377):
         k, v = C.run_gpu(c, gpu, g, samples=list(range(M - n, M)))
         assert torch.equal(k, kr[M - n:]) and torch.equal(v, vr[M - n:]), n
 
