@@ -10,6 +10,14 @@
 //   stream : 256 workgroups read a 1 GiB buffer in 32 MiB chunks (each XCD's 32 CUs split a chunk), in
 //            three modes: every XCD reads the same chunk sequence; every XCD reads its own chunks; XCD 0
 //            alone. Bandwidth per XCD and over the active XCDs.
+//   copy   : 256 workgroups, two waves each, copy fragments of 16 rows x 64 bytes (rows 512 bytes apart, as K and
+//            V of a prefix) into an LDS ring of 8 pages of 16 KB, two pages in flight per wave, with a lane's
+//            row and 16-byte chunk in MFMA order (row lane % 16, chunk lane / 16) or four neighbouring
+//            lanes to a row (copy_row and copy_chunk of fa_device.h). From the L2 (1 MiB per XCD, over and over)
+//            and from memory (32 MiB that eight workgroups of an XCD share, as the heads of a sample its K
+//            and V). The last page is compared with its source.
+//   lds    : 4 waves of one workgroup per CU read whole fragments back, 16 bytes per lane: in MFMA order, in
+//            the order of frag_slot (fa_device.h), and in that order without its rotation.
 // Every index is in bounds, every wait is capped (a side whose wait hits the cap stops), and only
 // workgroups 0 and the partner take part in a hand-off (the others return at once); the stream kernel
 // stores one word per workgroup at most.
@@ -116,6 +124,76 @@ __global__ void __launch_bounds__(256) stream(const unsigned char* W, unsigned l
   if (s == 0x12345678u) sink[blockIdx.x] = s;  // keeps the loads live
 }
 
+__device__ __forceinline__ int quad_row(int lane) { return lane >> 2; }
+__device__ __forceinline__ int quad_chunk(int lane) { return (lane ^ -(lane >> 4)) & 3; }
+__device__ __forceinline__ unsigned quad_slot(int lr, int lq) { return lr * 64 + ((lq ^ -(lr >> 2)) & 3) * 16; }
+
+constexpr int PAGE = 16384, RING = 8;
+extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
+
+__global__ void fill(unsigned* W, unsigned long long n) {
+  for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x; i < n;
+       i += (unsigned long long)gridDim.x * blockDim.x)
+    W[i] = (unsigned)i;
+}
+
+// W: 1 GiB of words that hold their index. L2: 256 pages of the XCD's own MiB, else 2048 of the eight workgroups'.
+template <bool L2>
+constexpr int kPages = L2 ? 256 : 2048;
+template <bool QUAD, bool L2>
+__global__ void __launch_bounds__(128) copy_order(const unsigned char* W, unsigned* bad) {
+  constexpr int PAGES = kPages<L2>;
+  const int x = blockIdx.x & 7, rk = blockIdx.x >> 3, lane = threadIdx.x & 63, lw = threadIdx.x >> 6;
+  const int row = QUAD ? quad_row(lane) : lane & 15, chunk = QUAD ? quad_chunk(lane) : lane >> 4;
+  auto src = [&](int pg) {  // of this wave: 16 rows x 512 bytes
+    const unsigned long long page = L2 ? x * 64ull + (pg + 2 * rk) % 64 : (x * 4ull + rk / 8) * PAGES + pg;
+    return W + page * PAGE + lw * 8192;
+  };
+  for (int pg = 0; pg < PAGES; pg++) {
+    const unsigned char* s = src(pg) + row * 512 + chunk * 16;
+    unsigned char* d = ring + (pg % RING) * PAGE + lw * 8192;
+#pragma unroll
+    for (int f = 0; f < 8; f++)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(s + f * 64),
+                                       (__attribute__((address_space(3))) void*)(d + f * 1024), 16, 0, 0);
+    __builtin_amdgcn_s_waitcnt(8 | (7 << 4) | (15 << 8));  // vmcnt(8): the page before has landed
+  }
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  // MFMA lane (lr, lq) of every fragment of the last page: row lr, chunk lq
+  const int lr = lane & 15, lq = lane >> 4;
+  const unsigned first = (unsigned)((src(PAGES - 1) - W) / 4);
+  unsigned wrong = 0;
+  for (int f = 0; f < 8; f++) {
+    const u32x4 v = *reinterpret_cast<const u32x4*>(ring + ((PAGES - 1) % RING) * PAGE + lw * 8192 + f * 1024 +
+                                                    (QUAD ? quad_slot(lr, lq) : lane * 16));
+    const unsigned want = first + lr * 128 + f * 16 + lq * 4;
+    wrong |= (v[0] != want) | (v[3] != want + 3);
+  }
+  if (wrong) atomicOr(bad, 1u);
+}
+
+// MODE 0 MFMA order, 1 frag_slot, 2 frag_slot without the rotation. 16 fragments per pass and wave.
+template <int MODE>
+__global__ void __launch_bounds__(256) lds_read(int passes, unsigned* sink) {
+  const int lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4;
+  for (int i = threadIdx.x; i < RING * PAGE / 4; i += 256) reinterpret_cast<unsigned*>(ring)[i] = i;
+  __syncthreads();
+  const unsigned at = (threadIdx.x >> 6) * 2 * PAGE + (MODE == 0 ? lane * 16 : MODE == 1 ? quad_slot(lr, lq) : lr * 64 + lq * 16);
+  u32x4 acc = {0, 0, 0, 0};
+  for (int p = 0; p < passes; p++) {
+    unsigned a = at + (p & 1) * PAGE;
+    asm volatile("" : "+v"(a));  // read anew in every pass
+    u32x4 v[16];
+#pragma unroll
+    for (int f = 0; f < 16; f++) v[f] = *reinterpret_cast<const u32x4*>(ring + a + f * 1024);
+#pragma unroll
+    for (int f = 0; f < 16; f++) acc ^= v[f];
+  }
+  const unsigned s = acc[0] ^ acc[1] ^ acc[2] ^ acc[3];
+  if (s == 0x12345678u) sink[blockIdx.x] = s;
+}
+
 int main() {
   unsigned char* buf = nullptr;
   unsigned long long* out = nullptr;
@@ -166,6 +244,52 @@ int main() {
     const int nx = mode == 2 ? 1 : 8;
     printf("stream %s: per_xcd_GBs %.0f total_GBs %.0f ms %.3f\n", names[mode], per_xcd / ms / 1e6,
            nx * per_xcd / ms / 1e6, ms);
+  }
+  auto timed = [&](auto launch) {  // ms of the second launch, negative on an error
+    float ms = -1.f;
+    for (int rep = 0; rep < 2; rep++) {
+      (void)hipEventRecord(a);
+      launch();
+      (void)hipEventRecord(b);
+      if (hipEventSynchronize(b) != hipSuccess || hipEventElapsedTime(&ms, a, b) != hipSuccess) return -1.f;
+    }
+    return ms;
+  };
+  static_assert(32ull * kPages<false> * PAGE == 1ull << 30, "the copies' pages are the buffer");
+  hipLaunchKernelGGL(fill, dim3(2048), dim3(256), 0, 0, reinterpret_cast<unsigned*>(W), size / 4);
+  unsigned wrong = 1;
+  if (hipMemset(sink, 0, 4) != hipSuccess) return 2;
+  const auto copies = {(const void*)copy_order<false, true>, (const void*)copy_order<true, true>,
+                       (const void*)copy_order<false, false>, (const void*)copy_order<true, false>};
+  const auto reads = {(const void*)lds_read<0>, (const void*)lds_read<1>, (const void*)lds_read<2>};
+  for (const void* k : copies)
+    if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, RING * PAGE) != hipSuccess) return 2;
+  for (const void* k : reads)
+    if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, RING * PAGE) != hipSuccess) return 2;
+  const char* cn[4] = {"l2 mfma-order", "l2 quad-order", "memory mfma-order", "memory quad-order"};
+  int i = 0;
+  for (const void* k : copies) {
+    const float ms = timed([&] {
+      const unsigned char* w = W;
+      void* args[] = {&w, &sink};
+      (void)hipLaunchKernel(k, dim3(256), dim3(128), args, RING * PAGE, 0);
+    });
+    if (ms <= 0.f) return 3;
+    printf("copy %s: per_cu_GBs %.1f\n", cn[i], (double)(i < 2 ? kPages<true> : kPages<false>) * PAGE / ms / 1e6);
+    i++;
+  }
+  if (hipMemcpy(&wrong, sink, 4, hipMemcpyDeviceToHost) != hipSuccess) return 3;
+  if (wrong) bad = 1;
+  const char* rn[3] = {"mfma-order", "rotated", "unrotated"};
+  i = 0;
+  for (const void* k : reads) {
+    int passes = 4000;
+    const float ms = timed([&] {
+      void* args[] = {&passes, &sink};
+      (void)hipLaunchKernel(k, dim3(256), dim3(256), args, RING * PAGE, 0);
+    });
+    if (ms <= 0.f) return 3;
+    printf("lds %s: per_cu_GBs %.0f\n", rn[i++], 4.0 * passes * PAGE / ms / 1e6);
   }
   unsigned h[256];
   if (hipMemcpy(h, xccs, sizeof(h), hipMemcpyDeviceToHost) != hipSuccess) return 3;
