@@ -152,11 +152,13 @@ size_t fa_pi05_workspace_bytes(int batch, int Tv, int Lmax);
 /* fa_pi05_denoise without a caller workspace. No counterpart in the reference: it is for callers
  * that cannot allocate device memory (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc). args->workspace must be NULL and workspace_bytes 0; the launch uses a
- * 16 MiB scratch the library reserves in device memory at load time (one per device, held until
+ * 16 MiB + 8 KiB scratch the library reserves in device memory at load time (one per device, held until
  * the process ends), zeroed by a fill kernel on `stream` at the first call on each device.
- * Requests whose workspace (fa_pi05_workspace_bytes) exceeds 16 MiB are rejected
- * (FA_ERR_INVALID_ARG); every batch-1 request fits. No hipMalloc, hipFree or other allocating call
- * is made. All calls on one device share the scratch, which keeps the last call's contents: calls
+ * Every batch-1 request fits. A batch fits if the stage-engine kernel's workspace does, and runs on that
+ * kernel: fa_pi05_workspace_bytes also makes room for the faster kernel that batches of 2 to 16 run on with
+ * a caller workspace (batch 2 at 968 + 50 tokens: 16.7 against 5.7 ms), which needs more than the
+ * scratch holds. Larger requests are rejected (FA_ERR_INVALID_ARG). No hipMalloc, hipFree or other
+ * allocating call is made. All calls on one device share the scratch, which keeps the last call's contents: calls
  * that overlap on one GPU race (serialise them on one stream, or use fa_pi05_denoise with one
  * workspace per concurrent call). *scratch_out (optional) receives the scratch's device address,
  * for fa_pi05_read_status and fa_pi05_workspace_init. */
@@ -167,8 +169,9 @@ size_t fa_pi05_cache_shadow_bytes(int batch, int num_layers, int Lmax);
 int fa_pi05_workspace_init(void* workspace, size_t bytes, fa_stream_t stream);
 /* Synchronous: copies the kernel status bits (FA_KSTATUS_*) of the last launch on this workspace. */
 int fa_pi05_read_status(const void* workspace, unsigned* status);
-/* Largest batch one launch accepts. batch 1 runs the latency-bound single-sample kernel, batch >= 2
- * the batched (MFMA-bound) kernel. The workspace size depends on the shape; one workspace that is
+/* Largest batch one launch accepts. batch 1 runs the latency-bound single-sample kernel, batches of 2 to 16
+ * the kernel of XCD groups, larger ones the stage-engine kernel (as do 9 to 16 samples with long prefixes,
+ * and workspaces with room for no more). The workspace size depends on the shape; one workspace that is
  * large enough may serve any sequence of launches of every entry point (never two at once). */
 int fa_pi05_max_batch(void);
 
