@@ -24,8 +24,8 @@
 //   [W] O     partial sums {E} N2 [W] GU [W] DN partial sums {E}
 //
 // What bounds it: each group streams all 34.6 MB of a layer's weights, 34.6/G MB per XCD. The fabric
-// feeds one XCD at 0.85-0.95 TB/s while all eight read (1.0 with four, 1.34 alone): 37 us per layer with
-// G = 1, 19 with G = 2, 10 with G = 4. The stage engine at these batches had 40 to 180 GEMM items for the 256
+// feeds one XCD at 0.80-0.97 TB/s while all eight read, 1.3 alone (tests/fabric_probe.hip): about 40 us per
+// layer with G = 1, 20 with G = 2, 10 with G = 4. The stage engine at these batches had 40 to 180 GEMM items for the 256
 // CUs in every stage but gate/up, and eight grid barriers of about 2 us per layer. At 16 samples a layer takes
 // 88 us: gate/up 20.7, attention 17.5 (its 512 KB of K/V per CU arrive at 44 GB/s; without softmax and P V it
 // takes as long), down 11.1, QKV 8.6, the norms 14.5 with the waits for the partial sums, barriers 5.7.
