@@ -377,9 +377,9 @@ __device__ __forceinline__ void proj24(const Params& p, const Ctx& c, const WF& 
   if (rt == 0 || c.lq < 2) {
     const int col = 24 * c.r + 16 * rt + 4 * c.lq;
     if (t >= p.Tv) acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    const uint32_t o = (uint32_t)(((c.g * TP + t) * D + col) * 4), xb = (uint32_t)(NX * TP * D * 4);
-    stb128<kCpSc1>(c.ws, kOffX<WHOLE> + buf * xb + o, WHOLE ? whole(acc) : tag(acc, par));
-    if (WHOLE) stb128<kCpSc1>(c.ws, kOffX<WHOLE> + (buf ^ 2) * xb + o, u32x4{~0u, ~0u, ~0u, ~0u});
+    auto slot = [&](int b) { return kOffX<WHOLE> + (uint32_t)((((b * NX + c.g) * TP + t) * D + col) * 4); };
+    __builtin_amdgcn_raw_buffer_store_b128(WHOLE ? whole(acc) : tag(acc, par), c.ws, slot(buf), 0, kCpSc1);
+    if (WHOLE) stb128<kCpSc1>(c.ws, slot(buf ^ 2), u32x4{~0u, ~0u, ~0u, ~0u});
   }
 }
 
